@@ -330,16 +330,16 @@ void plqcd_hip_server_destroy(plqcd_hip_server *s);
  *   order 0: block b -> tile b; 1: each XCD takes a contiguous eighth of the
  *   lattice; 2: XCDs sweep the lattice together, XCD k taking runs of `group`
  *   consecutive tiles; block: threads per block (64, 128, 256 or 512);
- *   tmarch > 0: full-lattice wilson applications whose time extent is a
- *   multiple of tmarch use the t-march kernel (one thread walks tmarch
- *   t-slices of a column), otherwise the one-site-per-thread gather kernel;
+ *   tmarch > 0: full-lattice applications use the t-march kernel (one thread
+ *   walks up to tmarch t-slices of a column: the time extent is cut into
+ *   balanced chunks), 0: the one-site-per-thread gather kernel;
  *   rb (1, 2 or 4): right-hand sides per thread of the gather kernel when it
  *   divides the field's RHS count (links are loaded once per rb RHS; the
  *   t-march kernel is used only with rb 1);
  *   tile_y, tile_z > 0: one-RHS t-march launches use the LDS-tiled kernel,
  *   whose blocks own tiles of L0 x tile_y x tile_z sites (both parities) and
  *   exchange neighbour spinors through LDS, when the tile divides the lattice
- *   and has 128 or 256 (or, below F64, 512) lanes = L0 tile_y tile_z
+ *   and has at most 256 (below F64, 512) lanes = L0 tile_y tile_z
  *   (block is then ignored); 0, 0: no tile.
  * Each RHS's result is bitwise the same for every launch shape.  Returns 0,
  * or nonzero for bad values. */

@@ -13,7 +13,7 @@ struct HopArgs {
    int order;    // block -> tile mapping (see logical_block)
    int group;    // blocks per XCD run for order 2
    int S;        // sites per parity in one t-slice (t-march)
-   int T;        // t-slices per thread (t-march)
+   int nt;       // chunks of the time extent (t-march, see chunk_t0)
    int R;        // right-hand sides per launch: lanes per site
    int r0;       // RHS of the fields that lane 0 of a site handles (the launch covers r0 .. r0+R-1)
    const int *rlist;     // when set: the launch covers RHS rlist[0 .. R-1] instead (device array)
@@ -27,19 +27,21 @@ struct HopArgs {
 // Launch shape of the hopping kernels, process-wide.
 struct HopTuning {
    int order, group, block;
-   int tmarch;  // t-slices per thread of the t-march kernel (0: gather kernel)
+   int tmarch;  // most t-slices per thread of the t-march kernel (0: gather kernel)
    int rb;      // right-hand sides per lane (1, 2 or 4; RHS-blocked gather when > 1)
    int ty, tz;  // LDS tile of the t-march (y and z extents; 0: untiled)
 };
 extern HopTuning g_tuning[3];  // per storage precision
 
 namespace plqcd {
-// Launch shape for `R` right-hand sides of storage format (prec, links) before
-// the per-shape cache: the precision's shape set by plqcd_hip_hop_tuning, else
-// a built-in default for R = 1 (per format) or for R > 1 (per precision), and
-// in both cases by whether the launch applies M = 1 - kappa H with or without
-// the CG update (`solver`) where that differs.
-HopTuning default_tuning(int prec, int links, int R, bool solver = false);
+// Launch shape for `R` right-hand sides of storage format (prec, links) on a
+// lattice with extents L before the per-shape cache of the autotuner: the
+// precision's shape set by plqcd_hip_hop_tuning, else the built-in rule's, by
+// whether the launch applies M = 1 - kappa H with or without the CG update
+// (`solver`).
+HopTuning default_tuning(const int L[4], int prec, int links, int R, bool solver = false);
+// The precision's shape set by plqcd_hip_hop_tuning, if one is.
+bool user_tuning(int prec, HopTuning *t);
 }  // namespace plqcd
 
 HopArgs make_hop_args(const plqcd_hip_lattice *lat, int parity);

@@ -2,75 +2,179 @@
 // per-format launchers (kernels in dslash_kernels.h, instantiated once per
 // storage precision and link format in dslash_<precision>_l<links>.hip), and the
 // process-wide launch shapes with the per-shape cache of the autotuner.
+#include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 
 #include "dslash.h"
+#include "reduce.h"
 
-// Built-in launch shapes, from sweeps at 32^3 x 64.  One RHS, per storage
-// format: the LDS-tiled t-march for F64 (tiles of 32 x 1 x 4 sites, 32
-// t-slices: 400 us with 18-real links against 414 us for 32 x 4 x 1 since
-// the x and one-plane z neighbour reads lost their per-lane test, and 434 us
-// for 32 x 4 x 1 and 514 us untiled before that; 12-real links: 331 us) and
-// F32 (32 x 1 x 4 sites
-// and 32 t-slices with 18-real links: 237 against 240 us for 32 x 8 x 1; 32 x
-// 8 x 2 and 8 t-slices with 12-real links: 168 against 176 us for 32 x 4 x
-// 4), for F16 with 18-real links 32 x 8 x 1 tiles over 4 t-slices in XCD runs
-// of 16 tiles (115 against 117 us for the untiled t-march), and with 12-real
-// links the untiled t-march over 8 t-slices in 512-lane blocks (90-102 us,
-// the gather kernel 116 us).  Shapes that do not
-// fit a lattice fall back to the untiled t-march or the gather kernel.  Several
-// RHS per launch, per precision: XCDs sweeping the lattice together, with
-// t-marches of 8 slices for F32/F16 (F16 at 12 RHS: 80 us per RHS, the
-// gather kernel 87 us) and 16 for F64 (which divides 48 as well as 32 and 64;
-// longer ones gain under 1 % at 32^3 x 64).
+// Built-in launch shapes.
+//
+// A march kernel's time is rounds x slices: its blocks run in rounds of as
+// many as the chip holds at once, and each block takes as many slice times as
+// its t-chunk has slices, plus a prologue worth `c` of them.  A last round
+// that is nearly empty costs almost as much as a full one, so the t-chunk
+// count that fits the rounds matters more than anything else in the shape: at
+// 24^3 x 48, F64 with one RHS on 24 x 4 x 2 tiles (192 lanes, one block per
+// CU), 16 slices per chunk fill 84 % of one round and take 153 us, 12 need a
+// second round and take 223 us.  The cost of a shape is therefore
+//
+//   lanes of a round x k x (slices + c) x (whole rounds + max(last round's share, f))
+//
+// and the cheapest shape is taken.  f is the share of a round below which the
+// blocks no longer run faster for being fewer (latency), k the kernel's time
+// per lane and slice relative to the others, `waves` how many waves of it a
+// SIMD's registers hold.  The gather kernel has no chunks and no rounds to
+// speak of.  The constants were fitted to timings of every shape of 8 lattices
+// from 8^3 x 16 to 32^3 x 64, 28 x 20 x 36 x 44 and 34 x 22 x 30 x 30 among
+// them, with one RHS, and of 6 lattices with 4 and 12 RHS; the shapes they
+// pick take on average 1.4 % (F64), 1-3 % (F32) and 1-3 % (F16) longer than
+// the fastest one timed, 16 % at most.
 namespace {
-struct FormatShape {
-   int prec, links;
-   HopTuning t;
+constexpr int kCus = 256;
+struct KernelCost {
+   int waves;
+   double k, f, c;
+   int most = 1 << 30;  // slices per chunk; blocks drift apart over long ones and lose their shared L2 lines
 };
-const FormatShape kOneRhs[6] = {{PLQCD_PREC_F64, 18, {1, 1, 256, 32, 1, 1, 4}},
-                                {PLQCD_PREC_F64, 12, {1, 1, 256, 32, 1, 1, 4}},
-                                {PLQCD_PREC_F32, 18, {1, 1, 256, 32, 1, 1, 4}},
-                                {PLQCD_PREC_F32, 12, {1, 1, 256, 8, 1, 8, 2}},
-                                {PLQCD_PREC_F16, 12, {1, 1, 512, 8, 1, 0, 0}},
-                                {PLQCD_PREC_F16, 18, {2, 16, 256, 4, 1, 8, 1}}};
-// One RHS with the solver epilogues (M with |Mp|^2, M^+ with the CG update),
-// where they differ from plain H: F64 18-real keeps 32 x 4 x 1 tiles (one CG
-// iteration's pair of launches 1.149 ms at 32^3 x 64; with 32 x 1 x 4 the
-// FP64 one-RHS solve took 0.0806 against 0.0769 s).
-const FormatShape kOneRhsSolver[1] = {{PLQCD_PREC_F64, 18, {1, 1, 256, 32, 1, 4, 1}}};
-const HopTuning kMultiRhs[3] = {{2, 8, 256, 16, 1, 0, 0}, {2, 8, 256, 8, 1, 0, 0}, {2, 8, 256, 8, 1, 0, 0}};
-// Several RHS with the solver epilogues (M, and M^+ with the residual
-// update): short t-marches.  F16 with 4-slice marches: the 12-RHS mixed CG at
-// 32^3 x 64 takes 0.2515 s against 0.256 s with the gather kernel, 1.24
-// against 1.36-1.40 s at 48^3 x 96.
-const HopTuning kMultiRhsSolver[3] = {{2, 8, 256, 16, 1, 0, 0}, {2, 8, 256, 4, 1, 0, 0}, {2, 8, 256, 4, 1, 0, 0}};
+struct FormatCost {
+   KernelCost march, tile, gather;
+};
+
+const FormatCost &one_rhs_cost(int prec, int links)
+{
+   static const FormatCost f64 = {{1, 1.05, 0.62, 0.13}, {1, 1.0, 0.90, 0.52}, {3, 1.57, 0.16, 0}};
+   static const FormatCost f32_18 = {{2, 1.02, 0.66, 0.12}, {2, 1.0, 0.51, 0.85}, {4, 1.52, 0.09, 0}};
+   static const FormatCost f32_12 = {{2, 1.13, 0.61, 0.11}, {2, 1.0, 0.97, 0.79}, {4, 1.55, 0.22, 0}};
+   static const FormatCost f16 = {{3, 0.97, 0.50, 0.27}, {2, 1.0, 0.74, 1.15}, {5, 1.10, 0.35, 0}};
+   return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F16 ? f16 : links == 18 ? f32_18 : f32_12;
+}
+
+const FormatCost &multi_rhs_cost(int prec)  // no tiles
+{
+   static const FormatCost f64 = {{1, 1.0, 0.98, 0.74, 32}, {}, {3, 1.35, 0.14, 0}};
+   static const FormatCost f32 = {{2, 1.0, 1.00, 1.44, 32}, {}, {4, 1.35, 0.32, 0}};
+   static const FormatCost f16 = {{3, 1.0, 0.83, 0.45, 12}, {}, {5, 1.30, 0.20, 0}};
+   return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F32 ? f32 : f16;
+}
+
+// LDS of a tile block (hop_tile_kernel): two slices of centre spinors, the
+// backward t terms and, in F64 blocks of up to 128 lanes, the x links.
+size_t tile_lds(int prec, int lanes)
+{
+   const int block = lanes <= 128 ? 128 : lanes <= 256 ? 256 : 512;
+   const size_t sp = prec == PLQCD_PREC_F64 ? 192 : prec == PLQCD_PREC_F32 ? 96 : 52;
+   const size_t hv = prec == PLQCD_PREC_F64 ? 96 : prec == PLQCD_PREC_F32 ? 48 : 52;
+   return block * (2 * sp + hv + (prec == PLQCD_PREC_F64 && block == 128 ? 144 : 0));
+}
+
+double rounds(double blocks, double resident, double f)
+{
+   const double x = blocks / resident, whole = std::floor(x);
+   return whole + (x > whole ? std::max(x - whole, f) : 0.0);
+}
+
+struct Pick {
+   const int *L;
+   HopTuning best{};
+   double cost = 1e300;
+   // `chunk_blocks` blocks per t-chunk, of `lanes` lanes, `per_cu` on a CU
+   void march(const KernelCost &c, HopTuning t, double chunk_blocks, int lanes, int per_cu)
+   {
+      for (int nt = (L[3] + std::min(c.most, L[3]) - 1) / std::min(c.most, L[3]); nt <= L[3];) {
+         const int T = (L[3] + nt - 1) / nt;
+         const double res = double(kCus) * per_cu;
+         t.tmarch = T;
+         offer(t, res * lanes * c.k * (T + c.c) * rounds(chunk_blocks * nt, res, c.f));
+         if (T == 1) break;
+         nt = (L[3] + T - 2) / (T - 1);  // the fewest chunks that are shorter
+      }
+   }
+   void offer(const HopTuning &t, double v)
+   {
+      if (v < cost * (1 - 1e-9)) {
+         cost = v;
+         best = t;
+      }
+   }
+};
+
+// The shape for R right-hand sides on the lattice with extents L.
+HopTuning pick_shape(const int L[4], int prec, int links, int R, bool solver)
+{
+   const int Lxh = L[0] / 2, wave = 64;
+   const double S = double(Lxh) * L[1] * L[2], Vh = S * L[3];
+   const FormatCost &fc = R <= 1 ? one_rhs_cost(prec, links) : multi_rhs_cost(prec);
+   Pick p{L};
+   // XCDs take contiguous eighths; with several RHS an eighth's slice no
+   // longer fits an XCD's L2 and the XCDs sweep the lattice together (F64, 12
+   // RHS at 32^3 x 64: 4.2 against 4.5 ms)
+   {
+      const int block = R <= 1 ? 64 : 256;
+      const int spb = REDUCE_CHUNK * std::max(1, block / (REDUCE_CHUNK * R));
+      const int lanes = spb * R, wpb = (lanes + wave - 1) / wave;
+      const HopTuning t{R <= 1 ? 1 : 2, R <= 1 ? 1 : 8, block, 0, 1, 0, 0};
+      const double res = double(kCus) * std::max(1, 4 * fc.gather.waves / wpb);
+      const double gb = 2 * std::ceil(Vh / spb);
+      p.offer(t, std::max(gb / res, fc.gather.f) * res * lanes * fc.gather.k);
+      p.march(fc.march, t, 2 * std::ceil(S / spb), lanes, std::max(1, 4 * fc.march.waves / wpb));
+   }
+   if (R <= 1) {
+      // tiles of 96 lanes or more; of two equally good ones plain H takes the
+      // flatter in y (F64 at 32^3 x 64: 401 us for 32 x 1 x 4, 414 for 32 x 4 x
+      // 1), the solver's epilogues the other (0.0769 against 0.0806 s a solve)
+      const int most = prec == PLQCD_PREC_F64 ? 256 : 512;
+      for (int i = 1; i <= L[1] && i * L[0] <= most; i++) {
+         for (int k = 1; k <= L[2] && k * L[0] <= most; k++) {
+            const int ty = i, tz = k, lanes = L[0] * ty * tz;
+            if (L[1] % ty || L[2] % tz || lanes < 96 || lanes > most) continue;
+            if (solver && Lxh * ty % REDUCE_CHUNK) continue;  // the norms' chunks
+            const int wpb = (lanes + wave - 1) / wave;
+            const int per_cu = std::min(4 * fc.tile.waves / wpb, int(160 * 1024 / tile_lds(prec, lanes)));
+            KernelCost c = fc.tile;
+            c.k *= 1 + 1e-6 * (solver ? tz : ty);
+            p.march(c, HopTuning{1, 1, 256, 0, 1, ty, tz}, S / (double(Lxh) * ty * tz), lanes, std::max(1, per_cu));
+         }
+      }
+   }
+   return p.best;
+}
 bool g_tuning_set[3] = {false, false, false};  // set by plqcd_hip_hop_tuning
 
-HopTuning one_rhs_shape(int prec, int links)
+HopTuning headline_shape(int prec)
 {
-   for (const FormatShape &f : kOneRhs)
-      if (f.prec == prec && f.links == links) return f.t;
-   for (const FormatShape &f : kOneRhs)
-      if (f.prec == prec) return f.t;
-   return kOneRhs[0].t;
+   const int L[4] = {32, 32, 32, 64};
+   return pick_shape(L, prec, prec == PLQCD_PREC_F16 ? 12 : 18, 1, false);
 }
+
+// Shapes picked so far, by value of what they were picked for.
+std::mutex g_shape_mu;
+std::map<plqcd::TuneKey, HopTuning> g_shapes;
+constexpr size_t kMostShapes = 4096;
 }  // namespace
 
-// The one-RHS shapes of the 18-real (F16: 12-real) formats, per precision;
-// plqcd_hip_hop_tuning replaces them.
-HopTuning g_tuning[3] = {one_rhs_shape(PLQCD_PREC_F64, 18), one_rhs_shape(PLQCD_PREC_F32, 18),
-                         one_rhs_shape(PLQCD_PREC_F16, 12)};
+// The one-RHS shapes at 32^3 x 64 of the 18-real (F16: 12-real) formats, per
+// precision; plqcd_hip_hop_tuning replaces them.
+HopTuning g_tuning[3] = {headline_shape(PLQCD_PREC_F64), headline_shape(PLQCD_PREC_F32),
+                         headline_shape(PLQCD_PREC_F16)};
 
-HopTuning plqcd::default_tuning(int prec, int links, int R, bool solver)
+bool plqcd::user_tuning(int prec, HopTuning *t)
+{
+   if (g_tuning_set[prec]) *t = g_tuning[prec];
+   return g_tuning_set[prec];
+}
+
+HopTuning plqcd::default_tuning(const int L[4], int prec, int links, int R, bool solver)
 {
    if (g_tuning_set[prec]) return g_tuning[prec];
-   if (R <= 1 && solver)
-      for (const FormatShape &f : kOneRhsSolver)
-         if (f.prec == prec && f.links == links) return f.t;
-   if (R <= 1) return one_rhs_shape(prec, links);
-   return solver ? kMultiRhsSolver[prec] : kMultiRhs[prec];
+   const TuneKey key{{L[0], L[1], L[2], L[3]}, prec, links, R, solver ? kTuneOpSolver : kTuneOpHop};
+   std::lock_guard<std::mutex> lk(g_shape_mu);
+   auto it = g_shapes.find(key);
+   if (it != g_shapes.end()) return it->second;
+   if (g_shapes.size() >= kMostShapes) g_shapes.clear();
+   return g_shapes[key] = pick_shape(L, prec, links, R, solver);
 }
 
 namespace {
@@ -136,7 +240,7 @@ HopArgs make_hop_args(const plqcd_hip_lattice *lat, int parity)
    a.order = 0;
    a.group = 1;
    a.S = lat->Vh / lat->L[3];
-   a.T = 1;
+   a.nt = 1;
    a.R = 1;
    a.spb = 256;
    return a;
@@ -211,7 +315,7 @@ extern "C" int plqcd_hip_hop_tuning_reset(int prec)
    if (prec < -1 || prec > PLQCD_PREC_F16) return plqcd::set_error(1, "plqcd_hip_hop_tuning_reset: bad precision");
    for (int p = 0; p < 3; p++)
       if (prec < 0 || p == prec) {
-         g_tuning[p] = one_rhs_shape(p, p == PLQCD_PREC_F16 ? 12 : 18);
+         g_tuning[p] = headline_shape(p);
          g_tuning_set[p] = false;
       }
    return 0;

@@ -395,21 +395,31 @@ __device__ __forceinline__ void hop_dir(const SIO &in, const GIO &g, int p, int 
 // the 8 XCDs round-robin (block b runs on XCD b % 8), and each XCD has its
 // own L2, so the order decides which L2 sees which part of the lattice:
 //   order 0: logical = b
-//   order 1: XCD k takes the k-th contiguous eighth of the lattice
+//   order 1: XCD k takes the k-th contiguous eighth of the lattice (eighths
+//            differ by one block where the block count is no multiple of 8)
 //   order 2: the lattice is cut into chunks of 8*group logical blocks; XCD k
 //            takes the k-th run of `group` blocks of every chunk, so all XCDs
-//            sweep the lattice together and neighbouring tiles share an L2
+//            sweep the lattice together and neighbouring tiles share an L2;
+//            the blocks after the last whole chunk are split as in order 1
+// Both are one-to-one for every block count.
 // The output parity alternates between consecutive logical blocks, so a link
 // is read as a forward and as a backward link by nearby tiles.
 __device__ __forceinline__ int logical_block(const HopArgs &a)
 {
-   const int b = blockIdx.x, nb = gridDim.x;
-   if (a.order == 1) return (b & 7) * (nb >> 3) + (b >> 3);
+   int b = blockIdx.x, nb = gridDim.x, first = 0;
+   if (a.order == 0) return b;
    if (a.order == 2) {
-      const int q = b >> 3, G = a.group;
-      return (q / G) * 8 * G + (b & 7) * G + (q % G);
+      const int G = a.group;
+      first = nb - nb % (8 * G);
+      if (b < first) {
+         const int q = b >> 3;
+         return (q / G) * 8 * G + (b & 7) * G + (q % G);
+      }
+      b -= first;
+      nb -= first;
    }
-   return b;
+   const int k = b & 7;
+   return first + k * (nb >> 3) + min(k, nb & 7) + (b >> 3);
 }
 
 // The RHS of the fields that lane-RHS r of a launch handles: r0 + r, or the
@@ -617,6 +627,14 @@ __global__ __launch_bounds__(BLOCK) void hop_rb_kernel(SIO in, SIO out, GIO g, H
    hop_block_rb<MODE, DAG, EPI, NORM, BLOCK, RB>(in, out, g, a, logical_block(a), f);
 }
 
+// First t-slice of t-chunk k of the marching kernels: the time extent is cut
+// into a.nt chunks whose lengths differ by at most one slice, so any chunk
+// count serves any extent.
+__device__ __forceinline__ int chunk_t0(const HopArgs &a, int k)
+{
+   return (int)((long long)k * a.L[3] / a.nt);
+}
+
 // One application of H on each of several independent lattices (each with its
 // own gauge field and fields) in a single launch over the concatenated
 // logical blocks of the items.
@@ -627,7 +645,6 @@ struct BatchItem {
    HopArgs a;
    int first;  // first global block of this item
    int nb;     // blocks of this item
-   int march;  // t-march blocks (a.T t-slices per lane) instead of gather blocks
 };
 // A launch takes up to kBatchItems items by value, as a kernel argument (no
 // device copy of the list); longer batches take several launches.
@@ -639,7 +656,8 @@ struct BatchList {
 };
 
 // t-march variant (full lattice, either mode): a thread owns one (x,y,z)
-// column and walks T consecutive t-slices.  Along t each spinor and each U_t
+// column and walks the consecutive t-slices of one of a.nt balanced chunks of
+// the time extent.  Along t each spinor and each U_t
 // is loaded once: psi(t+1), read as the forward t-neighbour at step t, is kept
 // (it is the centre site of step t+1) and its projection, multiplied by
 // U_t(t+1)^+ at step t+1 (that step's forward link), gives the backward
@@ -667,7 +685,7 @@ __device__ __forceinline__ void hop_tmarch_block(const SIO &in, const SO &out, c
    const SIO si = in.at_rhs(rr);
    const SO so = out.at_rhs(rr);
 
-   const int t0 = chunk * a.T;
+   const int t0 = chunk_t0(a, chunk), nts = chunk_t0(a, chunk + 1) - t0;
    const int cc = valid ? c : 0;
    const int row = cc / a.Lxh;  // y + L1*z
    const int xh = cc - row * a.Lxh;
@@ -751,7 +769,7 @@ __device__ __forceinline__ void hop_tmarch_block(const SIO &in, const SO &out, c
       term_udag<3, -SF>(f, u, b0);
       put_b(b0);
    }
-   for (int s = 0; s < a.T; s++) {
+   for (int s = 0; s < nts; s++) {
       const int t = t0 + s;
       const int p = q ^ (s & 1);
       const int base = t * S;
@@ -814,16 +832,14 @@ __global__ __launch_bounds__(BLOCK) void hop_tmarch_kernel(SIO in, SO out, GIO g
    hop_tmarch_block<MODE, DAG, EPI, NORM, BLOCK>(in, out, g, a, logical_block(a), fuse);
 }
 
-// One launch over a ragged batch (see BatchItem): each item runs t-march or
-// gather blocks.  Blocks go round-robin to the 8 XCDs; as in block order 2,
-// the XCDs sweep the concatenated logical blocks together, XCD k (blockIdx %
-// 8 == k) taking the k-th run of kBatchGroup consecutive blocks of every
-// 8 kBatchGroup.  The grid is a multiple of 8; a block takes logical blocks
-// at a stride of gridDim / 8 runs, so any such grid covers the batch (the
-// launch gives each logical block a block of its own).  KIND 0: every item runs gather blocks, 1:
-// every item t-march blocks, 2: each item its own kind (the kernel then holds
-// both code paths and needs the registers of the larger).
-template <int MODE, int KIND, int BLOCK, class SIO, class GIO>
+// One launch over a ragged batch (see BatchItem) of t-march blocks.  Blocks go
+// round-robin to the 8 XCDs; as in block order 2, the XCDs sweep the
+// concatenated logical blocks together, XCD k (blockIdx % 8 == k) taking the
+// k-th run of kBatchGroup consecutive blocks of every 8 kBatchGroup.  The grid
+// is a multiple of 8; a block takes logical blocks at a stride of gridDim / 8
+// runs, so any such grid covers the batch (the launch gives each logical block
+// a block of its own).
+template <int MODE, int BLOCK, class SIO, class GIO>
 __global__ __launch_bounds__(BLOCK) void hop_batch_kernel(const BatchList<SIO, GIO> items, int nitems, int total)
 {
    const int xcd = blockIdx.x & 7, per = gridDim.x >> 3;
@@ -834,16 +850,7 @@ __global__ __launch_bounds__(BLOCK) void hop_batch_kernel(const BatchList<SIO, G
       int it = 0;
       while (it + 1 < nitems && b >= items.it[it + 1].first) it++;
       const BatchItem<SIO, GIO> &I = items.it[it];
-      if constexpr (KIND == 1) {
-         hop_tmarch_block<MODE, false, 0, false, BLOCK>(I.in, I.out, I.g, I.a, b - I.first, CgFuse<SIO>{});
-      } else if constexpr (KIND == 2) {
-         if (I.march)
-            hop_tmarch_block<MODE, false, 0, false, BLOCK>(I.in, I.out, I.g, I.a, b - I.first, CgFuse<SIO>{});
-         else
-            hop_block<MODE, false, 0, false, BLOCK>(I.in, I.out, I.g, I.a, b - I.first, CgFuse<SIO>{});
-      } else {
-         hop_block<MODE, false, 0, false, BLOCK>(I.in, I.out, I.g, I.a, b - I.first, CgFuse<SIO>{});
-      }
+      hop_tmarch_block<MODE, false, 0, false, BLOCK>(I.in, I.out, I.g, I.a, b - I.first, CgFuse<SIO>{});
    }
 }
 
@@ -925,7 +932,7 @@ __device__ __forceinline__ void tile_dir(const SIO &in, const GIO &g, const type
 // LDS-tiled t-march (full lattice, one RHS).  A block owns the
 // columns of a tile of Lxh x ty x tz (x, y, z) sites -- whole x rows -- for
 // both parities: lanes q = 0 and 1 of a column hold its two x-adjacent sites,
-// and the block walks T t-slices.  The centre spinors of a t-slice are in LDS
+// and the block walks the t-slices of one t-chunk.  The centre spinors of a t-slice are in LDS
 // (two buffers, one barrier per slice), and the x, y and z
 // neighbours inside the tile are read from there; only the tile's y/z halo and
 // the t+1 spinor are loaded from memory.  The centre spinor and the backward
@@ -935,7 +942,7 @@ __device__ __forceinline__ void tile_dir(const SIO &in, const GIO &g, const type
 // second barrier per slice).  Terms are accumulated in the order of hop_kernel.
 // Compat mode takes the forward links of odd sites from the even site with
 // the same index (its t link with a second load, since the true one still
-// serves the next slice's backward term).  BLOCK = 2 Lxh ty tz lanes.
+// serves the next slice's backward term).  2 Lxh ty tz <= BLOCK lanes.
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, class SIO, class GIO>
 __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
 {
@@ -957,7 +964,7 @@ __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g,
    __shared__ typename GIO::U::E ux[XSH ? 9 : 1][XSH ? BLOCK : 1];  // the lanes' forward x links of this slice
    typedef typename GIO::U::E(*UxRow)[BLOCK];
    const int S = a.S;
-   constexpr int ncol = BLOCK / 2;
+   const int ncol = a.Lxh * a.ty * a.tz;  // columns of the tile, 2 ncol <= BLOCK lanes
    const int nty = a.L[1] / a.ty;
    const int ntile = nty * (a.L[2] / a.tz);
    const int lb = logical_block(a);
@@ -973,7 +980,7 @@ __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g,
    const int y = y0 + ly, z = z0 + lz;
    const int row = y + a.L[1] * z;
    const int c = row * a.Lxh + xh;
-   const int t0 = chunk * a.T;
+   const int t0 = chunk_t0(a, chunk), nts = chunk_t0(a, chunk + 1) - t0;
    const int x = 2 * xh + ((q + y + z + t0) & 1);  // the same at every t-slice
    const int sx = (1 - q) * ncol + lc;              // the lane with the same index j, other parity
    int cu[3], cd[3], su[3], sd[3];
@@ -1015,7 +1022,7 @@ __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g,
 #pragma unroll
       for (int m = 0; m < Hv::N; m++) sb[m][tid] = b.e[m];
    }
-   for (int s = 0; s < a.T; s++) {
+   for (int s = 0; s < nts; s++) {
       const int t = t0 + s;
       const int p = q ^ (s & 1);
       const int base = t * S;
@@ -1164,7 +1171,7 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
    a.r0 = op.nr > 0 && !op.rlist ? op.r0 : 0;
    a.rlist = op.rlist;
    const bool solver = op.kappa != nullptr;
-   HopTuning tu = plqcd::default_tuning(PREC, LINKS, R, solver);
+   HopTuning tu = plqcd::default_tuning(lat->L, PREC, LINKS, R, solver);
    plqcd::lookup_tuning(plqcd::TuneKey{{lat->L[0], lat->L[1], lat->L[2], lat->L[3]}, PREC, LINKS, R,
                                        solver ? plqcd::kTuneOpSolver : plqcd::kTuneOpHop},
                         &tu);
@@ -1207,36 +1214,32 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
       fu.p = spinor_io<PREC>(op.resid_b);
    }
    if (norm && a.nparity != 2) return plqcd::set_error(2, "hop: norms are only fused into full-lattice launches");
-   const int T = tu.tmarch;
-   // the t-march kernel serves full-lattice applications (either mode) whose
-   // time extent is a multiple of T (and, with a norm, whose t-slices hold
-   // whole reduction chunks)
-   const bool march = !centre && rb == 1 && T > 0 && a.nparity == 2 && lat->L[3] % T == 0 &&
-                      (!norm || a.S % REDUCE_CHUNK == 0);
+   // the t-march kernel serves full-lattice applications (either mode; with a
+   // norm, the t-slices hold whole reduction chunks), in t-chunks of at most
+   // tmarch slices
+   const bool march = !centre && rb == 1 && tu.tmarch > 0 && a.nparity == 2 && (!norm || a.S % REDUCE_CHUNK == 0);
    // the LDS-tiled t-march: one RHS, a tile of whole x rows dividing the y and
    // z extents, 2 Lxh ty tz lanes per block (at most 256 with F64 storage for
    // the LDS), and, with a norm, reduction chunks that do not leave a tile row
-   const int tlanes = 2 * lat->Lxh * tu.ty * tu.tz;
+   const long long tlanes = 2LL * lat->Lxh * tu.ty * tu.tz;
    const bool tiled = march && !resid && R == 1 && tu.ty > 0 && tu.tz > 0 && lat->L[1] % tu.ty == 0 &&
-                      lat->L[2] % tu.tz == 0 &&
-                      (tlanes == 128 || tlanes == 256 || (tlanes == 512 && PREC != PLQCD_PREC_F64)) &&
+                      lat->L[2] % tu.tz == 0 && tlanes <= (PREC == PLQCD_PREC_F64 ? 256 : 512) &&
                       (!norm || (lat->Lxh * tu.ty) % REDUCE_CHUNK == 0);
    const int variant = tiled ? V_TILE : march ? V_MARCH : (rb == 2 ? V_RB2 : rb == 4 ? V_RB4 : V_GATHER);
-   a.T = march ? T : 1;
+   a.nt = march ? (lat->L[3] + tu.tmarch - 1) / tu.tmarch : 1;
    int nb, nthreads = threads, mblock = maxblock;
    if (tiled) {
       a.ty = tu.ty;
       a.tz = tu.tz;
-      nb = (lat->L[1] / tu.ty) * (lat->L[2] / tu.tz) * (lat->L[3] / T);
-      nthreads = mblock = tlanes;
+      nb = (lat->L[1] / tu.ty) * (lat->L[2] / tu.tz) * a.nt;
+      nthreads = (int)tlanes;
+      mblock = nthreads <= 128 ? 128 : nthreads <= 256 ? 256 : 512;
    } else {
-      const int nblk = march ? ((a.S + a.spb - 1) / a.spb) * (lat->L[3] / T) : (lat->Vh + a.spb - 1) / a.spb;
+      const int nblk = march ? ((a.S + a.spb - 1) / a.spb) * a.nt : (lat->Vh + a.spb - 1) / a.spb;
       nb = nblk * a.nparity;
    }
-   // the remapped orders need whole rounds of 8 XCDs (and of 8*group blocks)
    a.order = tu.order;
    a.group = tu.group > 0 ? tu.group : 1;
-   if ((a.order == 1 && nb % 8) || (a.order == 2 && nb % (8 * a.group))) a.order = 0;
    const dim3 grid(nb), block(nthreads);
    hipStream_t st = lat->stream;
    int lrc = 0;
@@ -1298,27 +1301,31 @@ int launch_batch_t(int n, const plqcd_hip_gauge *const *g, const plqcd_hip_field
          const int R = in[i0 + i]->nrhs;
          block = std::max(block, REDUCE_CHUNK * (256 / (REDUCE_CHUNK * R)) * R);
       }
+      // t-chunks of 16 (F64) or 8 slices (or as plqcd_hip_hop_tuning asks),
+      // shorter ones while the batch has fewer blocks than the chip has places
+      int T = PREC == PLQCD_PREC_F64 ? 16 : 8;
+      HopTuning user{};
+      const bool asked = plqcd::user_tuning(PREC, &user) && user.tmarch > 0;
+      if (asked) T = user.tmarch;
       BatchList<S, G> L{};
-      int total = 0, nmarch = 0;
-      for (int i = 0; i < m; i++) {
-         BatchItem<S, G> &I = L.it[i];
-         I.in = spinor_io<PREC>(in[i0 + i]);
-         I.out = spinor_io<PREC>(out[i0 + i]);
-         I.g = gauge_io<PREC, LINKS>(g[i0 + i]);
-         const plqcd_hip_lattice *lat = g[i0 + i]->lat;
-         I.a = make_hop_args(lat, PLQCD_PARITY_ALL);
-         I.a.R = in[i0 + i]->nrhs;
-         I.a.spb = REDUCE_CHUNK * (block / (REDUCE_CHUNK * I.a.R));
-         // items march along t with the precision's t-slice count when it
-         // divides the time extent; the others use gather blocks
-         const int T = plqcd::default_tuning(PREC, LINKS, I.a.R).tmarch;
-         I.march = T > 0 && lat->L[3] % T == 0;
-         I.a.T = I.march ? T : 1;
-         I.nb = I.march ? 2 * ((I.a.S + I.a.spb - 1) / I.a.spb) * (lat->L[3] / T)
-                        : 2 * ((I.a.Vh + I.a.spb - 1) / I.a.spb);
-         I.first = total;
-         total += I.nb;
-         nmarch += I.march;
+      int total = 0;
+      for (;; T /= 2) {
+         total = 0;
+         for (int i = 0; i < m; i++) {
+            BatchItem<S, G> &I = L.it[i];
+            I.in = spinor_io<PREC>(in[i0 + i]);
+            I.out = spinor_io<PREC>(out[i0 + i]);
+            I.g = gauge_io<PREC, LINKS>(g[i0 + i]);
+            const plqcd_hip_lattice *lat = g[i0 + i]->lat;
+            I.a = make_hop_args(lat, PLQCD_PARITY_ALL);
+            I.a.R = in[i0 + i]->nrhs;
+            I.a.spb = REDUCE_CHUNK * (block / (REDUCE_CHUNK * I.a.R));
+            I.a.nt = (lat->L[3] + T - 1) / T;
+            I.nb = 2 * ((I.a.S + I.a.spb - 1) / I.a.spb) * I.a.nt;
+            I.first = total;
+            total += I.nb;
+         }
+         if (asked || T == 1 || total >= 512) break;
       }
       // one hardware block per logical block (8 XCDs x span, see
       // hop_batch_kernel): the hardware then balances the items' blocks over
@@ -1329,17 +1336,8 @@ int launch_batch_t(int n, const plqcd_hip_gauge *const *g, const plqcd_hip_field
          const int span = ((total + 8 * kBatchGroup - 1) / (8 * kBatchGroup)) * kBatchGroup;
          hipLaunchKernelGGL(kern, dim3(8 * span), dim3(block), 0, st, L, m, total);
       };
-      if (mode == PLQCD_HOP_COMPAT) {
-         if (nmarch == 0) go(hop_batch_kernel<PLQCD_HOP_COMPAT, 0, 256, S, G>);
-         else if (nmarch == m) go(hop_batch_kernel<PLQCD_HOP_COMPAT, 1, 256, S, G>);
-         else go(hop_batch_kernel<PLQCD_HOP_COMPAT, 2, 256, S, G>);
-      } else if (nmarch == 0) {
-         go(hop_batch_kernel<PLQCD_HOP_WILSON, 0, 256, S, G>);
-      } else if (nmarch == m) {
-         go(hop_batch_kernel<PLQCD_HOP_WILSON, 1, 256, S, G>);
-      } else {
-         go(hop_batch_kernel<PLQCD_HOP_WILSON, 2, 256, S, G>);
-      }
+      if (mode == PLQCD_HOP_COMPAT) go(hop_batch_kernel<PLQCD_HOP_COMPAT, 256, S, G>);
+      else go(hop_batch_kernel<PLQCD_HOP_WILSON, 256, S, G>);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return plqcd::set_error(10, "hop_batch: %s", hipGetErrorString(e));
    }

@@ -1,7 +1,7 @@
 // Autotuners of the hopping kernels' launch shape.
 //
 // For one (lattice, storage precision, link format, RHS count) they time every
-// candidate launch shape -- block->tile order (plain, contiguous per XCD, XCD
+// candidate launch shape -- the built-in rule's, and block->tile order (plain, contiguous per XCD, XCD
 // runs of 8 or 16 tiles), threads per block, t-march length (gather kernel or
 // T t-slices per thread, T dividing the time extent), right-hand sides per
 // lane (RHS-blocked gather) and, for one RHS, the LDS tile of the t-march
@@ -19,7 +19,7 @@
 
 namespace {
 
-std::vector<HopTuning> candidates(const plqcd_hip_gauge *g, const plqcd_hip_field *in)
+std::vector<HopTuning> candidates(const plqcd_hip_gauge *g, const plqcd_hip_field *in, bool solver)
 {
    const plqcd_hip_lattice *lat = g->lat;
    struct Cand {
@@ -30,7 +30,7 @@ std::vector<HopTuning> candidates(const plqcd_hip_gauge *g, const plqcd_hip_fiel
    std::vector<int> marches = {0};
    for (int T : {2, 4, 8, 16, 32})
       if (lat->L[3] % T == 0) marches.push_back(T);
-   std::vector<HopTuning> cands;
+   std::vector<HopTuning> cands = {plqcd::default_tuning(lat->L, g->prec, g->links, in->nrhs, solver)};
    for (int rb : {1, 2, 4}) {
       if (in->nrhs % rb) continue;
       for (int T : marches) {
@@ -73,11 +73,11 @@ extern "C" int plqcd_hip_autotune(const plqcd_hip_gauge *g, const plqcd_hip_fiel
    // the shapes of plain H applications; the solver's launches keep their own
    const plqcd::TuneKey key{{lat->L[0], lat->L[1], lat->L[2], lat->L[3]}, g->prec, g->links, in->nrhs,
                             plqcd::kTuneOpHop};
-   const std::vector<HopTuning> cands = candidates(g, in);
+   const std::vector<HopTuning> cands = candidates(g, in, false);
    HopTuning prev{};
    const bool had = plqcd::lookup_tuning(key, &prev);
    double best_t = 1e300;
-   HopTuning best_c = plqcd::default_tuning(g->prec, g->links, in->nrhs);
+   HopTuning best_c = plqcd::default_tuning(lat->L, g->prec, g->links, in->nrhs);
    hipEvent_t e0 = nullptr, e1 = nullptr;
    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
       if (e0) (void)hipEventDestroy(e0);
@@ -176,12 +176,12 @@ extern "C" int plqcd_hip_autotune_solver(const plqcd_hip_gauge *g, const plqcd_h
    HopTuning prev{};
    const bool had = plqcd::lookup_tuning(key, &prev);
    double best_t = 1e300;
-   HopTuning best_c = plqcd::default_tuning(g->prec, g->links, R, true);
+   HopTuning best_c = plqcd::default_tuning(lat->L, g->prec, g->links, R, true);
    hipEvent_t e0 = nullptr, e1 = nullptr;
    if (!rc && hipEventCreate(&e0) != hipSuccess) rc = plqcd::set_error(10, "autotune_solver: hipEventCreate");
    if (!rc && hipEventCreate(&e1) != hipSuccess) rc = plqcd::set_error(10, "autotune_solver: hipEventCreate");
    if (!rc) {
-      for (const HopTuning &c : candidates(g, in)) {
+      for (const HopTuning &c : candidates(g, in, true)) {
          plqcd::store_tuning(key, c);
          rc = pair();  // warm-up
          if (rc == 2) {  // no kernel of this shape for the fused epilogues: not a candidate

@@ -1,0 +1,106 @@
+"""Launch shapes on extents that divide nothing: block orders over any block
+count, balanced t-chunks, partly filled tile blocks, and the built-in rule's
+own shapes.  Every kernel variant applies the same operations in the same
+order, so each result is bitwise the gather kernel's in plain block order;
+that one is held to the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = {0: 1e-13, 1: 2e-6, 2: 4e-3}  # as the hopping tests: storage precision F64, F32, F16
+
+
+@pytest.fixture(scope="module")
+def hp():
+    from plqcd_amd import hopping
+    return hopping
+
+
+def set_shape(prec, shape):
+    from plqcd_amd import capi
+    if shape is None:
+        assert capi.lib().plqcd_hip_hop_tuning_reset(prec) == 0
+    else:
+        assert capi.lib().plqcd_hip_hop_tuning(prec, *shape) == 0
+
+
+def fields(hp, L, prec, links, R):
+    V = int(np.prod(L))
+    lat = hp.Lattice(L)
+    u = hp.random_gauge_su3(V, 5)
+    g = hp.Gauge(lat, prec, links).upload(u)
+    fi, fo = hp.Field(lat, prec, R), hp.Field(lat, prec, R)
+    qs = [hp.random_spinor(V, 50 + r) for r in range(R)]
+    for r, q in enumerate(qs):
+        fi.upload(q, r)
+    return lat, g, fi, fo, qs, u
+
+
+# order, group, block, tmarch, rb, tile_y, tile_z
+SHAPES = [(1, 1, 64, 0, 1, 0, 0), (2, 8, 64, 0, 1, 0, 0), (2, 3, 128, 0, 1, 0, 0), (1, 1, 64, 1, 1, 0, 0),
+          (2, 8, 64, 3, 1, 0, 0), (1, 1, 128, 4, 1, 0, 0), (2, 5, 64, 7, 1, 0, 0), (1, 1, 256, 64, 1, 0, 0), None]
+TILES = [(1, 1, 256, 3, 1, 3, 1), (2, 8, 256, 4, 1, 3, 2), (1, 1, 256, 5, 1, 1, 7), (0, 1, 256, 64, 1, 6, 1)]
+
+
+@pytest.mark.parametrize("L", [(4, 6, 14, 10), (10, 6, 14, 6)])
+@pytest.mark.parametrize("prec,links,R", [(0, 18, 1), (1, 12, 1), (2, 18, 1), (0, 12, 3), (1, 18, 5), (2, 12, 12)])
+def test_shapes_on_ragged_extents(hp, L, prec, links, R):
+    import oracle
+    lat, g, fi, fo, qs, u = fields(hp, L, prec, links, R)
+    try:
+        for mode in (hp.HOP_WILSON, hp.HOP_COMPAT):
+            set_shape(prec, (0, 1, 256, 0, 1, 0, 0))
+            hp.hop(g, fi, fo, hp.PARITY_ALL, mode)
+            want = [fo.download(r) for r in range(R)]
+            ref = oracle.hopping_full(qs[-1], u, L, mode)
+            assert np.abs(want[-1] - ref).max() <= TOL[prec] * np.abs(ref).max()
+            for shape in SHAPES + (TILES if R == 1 else []):
+                set_shape(prec, shape)
+                for r in range(R):
+                    fo.upload(np.zeros_like(qs[0]), r)
+                hp.hop(g, fi, fo, hp.PARITY_ALL, mode)
+                for r in range(R):
+                    assert np.array_equal(fo.download(r), want[r]), (mode, shape, r)
+    finally:
+        set_shape(prec, None)
+
+
+def test_solver_shapes_on_ragged_extents(hp):
+    """The norms' reduction chunks over balanced t-chunks and partly filled
+    tiles: a solve takes the same iterates to the same bits."""
+    from plqcd_amd import solver
+    L = (8, 6, 10, 14)
+    lat, g, b, x, qs, u = fields(hp, L, hp.PREC_F64, 18, 1)
+    want = None
+    try:
+        for shape in ((0, 1, 256, 0, 1, 0, 0), (1, 1, 128, 5, 1, 0, 0), (1, 1, 256, 3, 1, 2, 5), None):
+            set_shape(hp.PREC_F64, shape)
+            st = solver.cg_solve(g, b, x, 0.12, 1e-10)
+            got = (st[0]["iterations"], st[0]["true_residual"], x.download())
+            assert st[0]["converged"]
+            if want is None:
+                want = got
+            assert got[:2] == want[:2] and np.array_equal(got[2], want[2]), shape
+    finally:
+        set_shape(hp.PREC_F64, None)
+
+
+def test_batch_of_small_ragged_lattices(hp):
+    """Every item of a batch is bitwise its own launch."""
+    shapes = [(4, 6, 14, 10), (4, 4, 4, 4), (6, 10, 4, 22)]
+    sets = [fields(hp, L, hp.PREC_F32, 12, R) for L, R in zip(shapes, (4, 1, 12))]
+    stream = hp.lib().plqcd_hip_lattice_stream(sets[0][0].h)
+    for s in sets:
+        s[0].set_stream(stream)
+    for mode in (hp.HOP_WILSON, hp.HOP_COMPAT):
+        want = []
+        for lat, g, fi, fo, qs, u in sets:
+            hp.hop(g, fi, fo, hp.PARITY_ALL, mode)
+            want.append([fo.download(r) for r in range(fo.nrhs)])
+            for r in range(fo.nrhs):
+                fo.upload(np.zeros_like(qs[0]), r)
+        hp.hop_batch([s[1] for s in sets], [s[2] for s in sets], [s[3] for s in sets], mode)
+        for s, w in zip(sets, want):
+            for r in range(s[3].nrhs):
+                assert np.array_equal(s[3].download(r), w[r]), (s[0].L, mode, r)
