@@ -19,6 +19,7 @@ struct HopArgs {
    const int *rlist;     // when set: the launch covers RHS rlist[0 .. R-1] instead (device array)
    int spb;      // sites per block
    int ty, tz;   // tile extents in y and z (LDS-tiled kernel)
+   int gy, gz;   // column blocks of a patch in y and z (pipelined t-march; gy 0: no patches)
    int nchunk;   // reduction chunks per parity
    const double *kappa;  // per-RHS kappa of M = 1 - kappa H (EPI = 1)
    double *partial;      // [R][2*nchunk] chunk sums of |out|^2 (NORM)
@@ -30,6 +31,7 @@ struct HopTuning {
    int tmarch;  // most t-slices per thread of the t-march kernel (0: gather kernel)
    int rb;      // right-hand sides per lane (1, 2 or 4; RHS-blocked gather when > 1)
    int ty, tz;  // LDS tile of the t-march (y and z extents; 0: untiled)
+   int gy = 0, gz = 0;  // patches of the pipelined t-march (built-in shapes only)
 };
 extern HopTuning g_tuning[3];  // per storage precision
 

@@ -30,10 +30,11 @@
 // speak of.  The constants were fitted to timings of every shape of 8 lattices
 // from 8^3 x 16 to 32^3 x 64, 28 x 20 x 36 x 44 and 34 x 22 x 30 x 30 among
 // them, with one RHS, and of 6 lattices with 4 and 12 RHS; the shapes they
-// pick take on average 1.4 % (F64), 1-3 % (F32) and 1-3 % (F16) longer than
+// pick take on average 0-1.4 % (F64), 1-3 % (F32) and 1-3 % (F16) longer than
 // the fastest one timed, 16 % at most.
 namespace {
 constexpr int kCus = 256;
+constexpr int kPipeRhs = 4;  // right-hand sides from which the pipelined t-march runs (pipe_fits)
 struct KernelCost {
    int waves;
    double k, f, c;
@@ -52,12 +53,53 @@ const FormatCost &one_rhs_cost(int prec, int links)
    return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F16 ? f16 : links == 18 ? f32_18 : f32_12;
 }
 
-const FormatCost &multi_rhs_cost(int prec)  // no tiles
+const FormatCost &multi_rhs_cost(int prec, int R)  // no tiles
 {
+   // the t-march (2 and 3 RHS)
    static const FormatCost f64 = {{1, 1.0, 0.98, 0.74, 32}, {}, {3, 1.35, 0.14, 0}};
    static const FormatCost f32 = {{2, 1.0, 1.00, 1.44, 32}, {}, {4, 1.35, 0.32, 0}};
    static const FormatCost f16 = {{3, 1.0, 0.83, 0.45, 12}, {}, {5, 1.30, 0.20, 0}};
-   return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F32 ? f32 : f16;
+   // the pipelined t-march
+   static const FormatCost p64 = {{1, 1.0, 0.99, 0.97, 32}, {}, {3, 1.57, 0.37, 0}};
+   static const FormatCost p32 = {{2, 1.0, 0.78, 0.80, 32}, {}, {4, 1.49, 0.39, 0}};
+   static const FormatCost p16 = {{3, 1.0, 0.92, 0.20, 12}, {}, {5, 1.40, 0.16, 0}};
+   if (R < kPipeRhs) return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F32 ? f32 : f16;
+   return prec == PLQCD_PREC_F64 ? p64 : prec == PLQCD_PREC_F32 ? p32 : p16;
+}
+
+// LDS of a pipelined t-march block (hop_pipe_block): two slices' links
+size_t pipe_lds(int prec, int spb)
+{
+   return size_t(14) * spb * (prec == PLQCD_PREC_F64 ? 144 : prec == PLQCD_PREC_F32 ? 80 : 48);
+}
+
+// The patch of gy x gz column blocks (of spb sites each, both parities) that
+// an XCD's L2 serves at a time: the least halo per site -- 1 / rows in y and 1
+// / planes in z, none over a whole extent -- of the patches with at most as
+// many column blocks as an XCD holds and its L2 keeps the slices of (F64 16,
+// else 48; 24^3 x 48, 12 RHS: F64 12 blocks 1032 us, 18 1038, 24 1064, 36 1078;
+// F32 24 blocks 499 us, 36 494, 48 491; 32^3 x 64 F16 32 blocks 894, 64 909).
+void pick_patch(const int L[4], int prec, int spb, HopTuning *t)
+{
+   const int Lxh = L[0] / 2, nby = Lxh * L[1] / spb, most = prec == PLQCD_PREC_F64 ? 16 : 48;
+   t->order = 1;
+   t->group = 1;
+   if (nby < 1 || Lxh * L[1] % spb) return;
+   double best = 1e300;
+   for (int gy = 1; gy <= nby && gy <= most; gy++) {
+      if (nby % gy) continue;
+      for (int gz = 1; gz <= L[2] && gy * gz <= most; gz++) {
+         if (L[2] % gz) continue;
+         const double halo = (gy < nby ? double(Lxh) / (gy * spb) : 0) + (gz < L[2] ? 1.0 / gz : 0) + 1e-6 * gy * gz;
+         if (halo < best) {
+            best = halo;
+            t->gy = gy;
+            t->gz = gz;
+         }
+      }
+   }
+   t->order = 2;
+   t->group = 2 * t->gy * t->gz;
 }
 
 // LDS of a tile block (hop_tile_kernel): two slices of centre spinors, the
@@ -106,20 +148,29 @@ HopTuning pick_shape(const int L[4], int prec, int links, int R, bool solver)
 {
    const int Lxh = L[0] / 2, wave = 64;
    const double S = double(Lxh) * L[1] * L[2], Vh = S * L[3];
-   const FormatCost &fc = R <= 1 ? one_rhs_cost(prec, links) : multi_rhs_cost(prec);
+   const FormatCost &fc = R <= 1 ? one_rhs_cost(prec, links) : multi_rhs_cost(prec, R);
    Pick p{L};
-   // XCDs take contiguous eighths; with several RHS an eighth's slice no
-   // longer fits an XCD's L2 and the XCDs sweep the lattice together (F64, 12
-   // RHS at 32^3 x 64: 4.2 against 4.5 ms)
-   {
-      const int block = R <= 1 ? 64 : 256;
+   // one RHS: each XCD takes a contiguous eighth; with several an eighth's
+   // slice no longer fits an XCD's L2 and the XCDs sweep the lattice together
+   // (t-march, F64, 12 RHS at 32^3 x 64: 4.2 against 4.5 ms)
+   for (int block : {64, 128, 256}) {
+      if (R <= 1 ? block != 64 : R < kPipeRhs ? block != 256 : block == 64) continue;
       const int spb = REDUCE_CHUNK * std::max(1, block / (REDUCE_CHUNK * R));
       const int lanes = spb * R, wpb = (lanes + wave - 1) / wave;
-      const HopTuning t{R <= 1 ? 1 : 2, R <= 1 ? 1 : 8, block, 0, 1, 0, 0};
+      HopTuning t{R <= 1 ? 1 : 2, R <= 1 ? 1 : 8, block, 0, 1, 0, 0};
       const double res = double(kCus) * std::max(1, 4 * fc.gather.waves / wpb);
       const double gb = 2 * std::ceil(Vh / spb);
       p.offer(t, std::max(gb / res, fc.gather.f) * res * lanes * fc.gather.k);
-      p.march(fc.march, t, 2 * std::ceil(S / spb), lanes, std::max(1, 4 * fc.march.waves / wpb));
+      int per_cu = 4 * fc.march.waves / wpb;
+      if (R >= kPipeRhs) {
+         per_cu = std::min<int>(per_cu, 160 * 1024 / pipe_lds(prec, spb));
+         pick_patch(L, prec, spb, &t);
+      }
+      // smaller blocks share each link and halo row among fewer lanes: only
+      // where they fit the rounds clearly better
+      KernelCost c = fc.march;
+      if (R >= kPipeRhs && block == 128) c.k *= 1.1;
+      p.march(c, t, 2 * std::ceil(S / spb), lanes, std::max(1, per_cu));
    }
    if (R <= 1) {
       // tiles of 96 lanes or more; of two equally good ones plain H takes the

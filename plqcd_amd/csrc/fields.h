@@ -36,6 +36,19 @@ __device__ __forceinline__ T ld(const char *ubase, uint32_t off)
    else
       return *reinterpret_cast<const T *>(ubase + off);
 }
+// The same load with ubase in a scalar-register pair that the compiler does
+// not see through, so that it cannot fold the lane's offset into it.  For
+// kernels that load many components at few site offsets in a loop, whose
+// per-lane addresses would otherwise be strength-reduced into two registers
+// for each component and neighbour.  ubase must be wave-uniform.
+template <class T>
+__device__ __forceinline__ T ld_s(const char *ubase, uint32_t off)
+{
+   typedef const __attribute__((address_space(1))) char *global_ptr;
+   global_ptr b = (global_ptr)ubase;
+   asm volatile("" : "+s"(b));
+   return *reinterpret_cast<const __attribute__((address_space(1))) T *>(b + off);
+}
 template <class T>
 __device__ __forceinline__ void st_nt(char *ubase, uint32_t off, T v)
 {
@@ -127,6 +140,21 @@ struct SpinorIO<PLQCD_PREC_F64> {
       for (int c = 0; c < 12; c++) st_nt(const_cast<char *>(cbase(parity, c)), o, s[c]);
    }
    __device__ __forceinline__ void load_sp(int parity, int j, Sp &s) const { load(parity, j, s.e); }
+   // load_sp on scalar component bases (parity wave-uniform)
+   __device__ __forceinline__ void load_sps(int parity, int j, Sp &s) const
+   {
+      const uint32_t o = off(j);
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+         if constexpr (NC == 12) {
+            s.e[c] = ld_s<C>(cbase(parity, c), o);
+         } else {
+            const f4 v = ld_s<f4>(cbase(parity, c), o);
+            s.e[2 * c] = C{v.x, v.y};
+            s.e[2 * c + 1] = C{v.z, v.w};
+         }
+      }
+   }
    static __device__ __forceinline__ void to_c(const Sp &s, C c[12])
    {
 #pragma unroll
@@ -173,6 +201,21 @@ struct SpinorIO<PLQCD_PREC_F32> {
          st_nt(const_cast<char *>(cbase(parity, c)), o, f4{s[2 * c].x, s[2 * c].y, s[2 * c + 1].x, s[2 * c + 1].y});
    }
    __device__ __forceinline__ void load_sp(int parity, int j, Sp &s) const { load(parity, j, s.e); }
+   // load_sp on scalar component bases (parity wave-uniform)
+   __device__ __forceinline__ void load_sps(int parity, int j, Sp &s) const
+   {
+      const uint32_t o = off(j);
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+         if constexpr (NC == 12) {
+            s.e[c] = ld_s<C>(cbase(parity, c), o);
+         } else {
+            const f4 v = ld_s<f4>(cbase(parity, c), o);
+            s.e[2 * c] = C{v.x, v.y};
+            s.e[2 * c + 1] = C{v.z, v.w};
+         }
+      }
+   }
    static __device__ __forceinline__ void to_c(const Sp &s, C c[12])
    {
 #pragma unroll
@@ -220,6 +263,19 @@ struct SpinorIO<PLQCD_PREC_F16> {
          s.e[4 * q + 2] = w.z;
          s.e[4 * q + 3] = w.w;
       }
+   }
+   __device__ __forceinline__ void load_sps(int parity, int j, Sp &s) const
+   {
+      const uint32_t o = off(j);
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+         const u4 w = ld_s<u4>(cbase(parity, q), o);
+         s.e[4 * q + 0] = w.x;
+         s.e[4 * q + 1] = w.y;
+         s.e[4 * q + 2] = w.z;
+         s.e[4 * q + 3] = w.w;
+      }
+      s.e[12] = ld_s<uint32_t>(sbase + parity * spstride, soff(j));
    }
    static __device__ __forceinline__ void to_c(const Sp &s, C c[12])
    {
@@ -306,7 +362,9 @@ inline SpinorIO<PREC> spinor_io(const plqcd_hip_field *f)
 //
 // load_u(parity, mu, j, u) reads the link U_mu of site j of `parity` into its
 // held form; load_u<true> does the same with streaming (non-temporal) loads,
-// for a link that only the loading lane reads.
+// for a link that only the loading lane reads.  load_raw reads only the stored
+// elements and finish completes the held form from them (row 2 of 12-real
+// links), so that a kernel can have the loads in flight while it works.
 
 template <int PREC, int LINKS>
 struct GaugeIO;
@@ -318,17 +376,20 @@ struct GaugeIO<PLQCD_PREC_F64, 18> {
    const char *base;
    size_t kstride;  // Vh*16: bytes between link components
    template <bool NT = false>
-   __device__ __forceinline__ void load(int parity, int mu, int j, C u[9]) const
+   __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
+      C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 9 * kstride;
       const uint32_t o = (uint32_t)j * 16;
 #pragma unroll
       for (int k = 0; k < 9; k++) u[k] = ld<d2, NT>(b + k * kstride, o);
    }
+   static __device__ __forceinline__ void finish(U &) {}
    template <bool NT = false>
    __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
    {
-      load<NT>(parity, mu, j, u.e);
+      load_raw<NT>(parity, mu, j, u);
+      finish(u);
    }
 };
 
@@ -339,18 +400,20 @@ struct GaugeIO<PLQCD_PREC_F64, 12> {
    const char *base;
    size_t kstride;
    template <bool NT = false>
-   __device__ __forceinline__ void load(int parity, int mu, int j, C u[9]) const
+   __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
+      C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 6 * kstride;
       const uint32_t o = (uint32_t)j * 16;
 #pragma unroll
       for (int k = 0; k < 6; k++) u[k] = ld<d2, NT>(b + k * kstride, o);
-      reconstruct_row2(u);
    }
+   static __device__ __forceinline__ void finish(U &u) { reconstruct_row2(u.e); }
    template <bool NT = false>
    __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
    {
-      load<NT>(parity, mu, j, u.e);
+      load_raw<NT>(parity, mu, j, u);
+      finish(u);
    }
 };
 
@@ -361,17 +424,20 @@ struct GaugeIO<PLQCD_PREC_F32, 18> {
    const char *base;
    size_t kstride;  // Vh*8
    template <bool NT = false>
-   __device__ __forceinline__ void load(int parity, int mu, int j, C u[9]) const
+   __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
+      C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 9 * kstride;
       const uint32_t o = (uint32_t)j * 8;
 #pragma unroll
       for (int k = 0; k < 9; k++) u[k] = ld<f2, NT>(b + k * kstride, o);
    }
+   static __device__ __forceinline__ void finish(U &) {}
    template <bool NT = false>
    __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
    {
-      load<NT>(parity, mu, j, u.e);
+      load_raw<NT>(parity, mu, j, u);
+      finish(u);
    }
 };
 
@@ -382,8 +448,9 @@ struct GaugeIO<PLQCD_PREC_F32, 12> {
    const char *base;
    size_t kstride;  // Vh*16
    template <bool NT = false>
-   __device__ __forceinline__ void load(int parity, int mu, int j, C u[9]) const
+   __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
+      C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 3 * kstride;
       const uint32_t o = (uint32_t)j * 16;
 #pragma unroll
@@ -392,12 +459,13 @@ struct GaugeIO<PLQCD_PREC_F32, 12> {
          u[2 * k] = f2{v.x, v.y};
          u[2 * k + 1] = f2{v.z, v.w};
       }
-      reconstruct_row2(u);
    }
+   static __device__ __forceinline__ void finish(U &u) { reconstruct_row2(u.e); }
    template <bool NT = false>
    __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
    {
-      load<NT>(parity, mu, j, u.e);
+      load_raw<NT>(parity, mu, j, u);
+      finish(u);
    }
 };
 
@@ -459,7 +527,7 @@ struct GaugeIO<PLQCD_PREC_F16, 12> {
    const char *base;  // [parity][mu][Vh] u4 (u00,u01,u02,u10), then [parity][mu][Vh] u2 (u11,u12)
    size_t kstride;    // Vh*16
    template <bool NT = false>
-   __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
+   __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &u) const
    {
       const size_t slot = (size_t)(parity * 4 + mu);
       const u4 a = ld<u4, NT>(base + slot * kstride, (uint32_t)j * 16);
@@ -470,7 +538,13 @@ struct GaugeIO<PLQCD_PREC_F16, 12> {
       u.e[3] = a.w;
       u.e[4] = b.x;
       u.e[5] = b.y;
-      row2_h(u.e);
+   }
+   static __device__ __forceinline__ void finish(U &u) { row2_h(u.e); }
+   template <bool NT = false>
+   __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
+   {
+      load_raw<NT>(parity, mu, j, u);
+      finish(u);
    }
 };
 
@@ -481,7 +555,7 @@ struct GaugeIO<PLQCD_PREC_F16, 18> {
    const char *base;  // [parity][mu][Vh] u4 (u00..u10), u4 (u11..u21), then [parity][mu][Vh] u32 (u22)
    size_t kstride;    // Vh*16
    template <bool NT = false>
-   __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
+   __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &u) const
    {
       const size_t slot = (size_t)(parity * 4 + mu);
       const u4 a = ld<u4, NT>(base + slot * kstride, (uint32_t)j * 16);
@@ -495,6 +569,12 @@ struct GaugeIO<PLQCD_PREC_F16, 18> {
       u.e[6] = b.z;
       u.e[7] = b.w;
       u.e[8] = ld<uint32_t, NT>(base + 16 * kstride + slot * (kstride / 4), (uint32_t)j * 4);
+   }
+   static __device__ __forceinline__ void finish(U &) {}
+   template <bool NT = false>
+   __device__ __forceinline__ void load_u(int parity, int mu, int j, U &u) const
+   {
+      load_raw<NT>(parity, mu, j, u);
    }
 };
 
