@@ -10,7 +10,8 @@ struct HopArgs {
    int Vh;       // sites per parity
    int nparity;  // 1 (eo or oe) or 2 (full H)
    int parity0;  // output parity when nparity == 1
-   int order;    // block -> tile mapping (see logical_block)
+   int order;    // block -> tile mapping (see logical_block; 3: hop_half_kernel)
+   int stream_links;  // hop_half_kernel: streaming link loads
    int group;    // blocks per XCD run for order 2
    int S;        // sites per parity in one t-slice (t-march)
    int nt;       // chunks of the time extent (t-march, see chunk_t0)
@@ -59,7 +60,7 @@ namespace plqcd {
 //                    the residual), whose |out|^2 goes to partial
 //   centre  != null: (with kappa; no dag, norm, alpha or resid_b) out = centre -
 //                    kappa[r] * (H in) on the output parity, the centre read
-//                    from that field rather than from in (gather kernel)
+//                    from that field rather than from in (one parity only)
 //   resid_b != null: residual (with dag, kappa and partial; F64 storage):
 //                    out = resid_b - (in - kappa H^+ in) for every RHS of the
 //                    launch, stored in out's own precision (any), and its |out|^2

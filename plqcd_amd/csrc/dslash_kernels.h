@@ -356,7 +356,8 @@ __device__ __forceinline__ void accum(f2 acc[12], const HalfH &r)
 // H uses (1 - gamma_mu) forward and (1 + gamma_mu) backward; the adjoint
 // H^+ = gamma5 H gamma5 has the signs swapped (gamma5 anticommutes with
 // gamma_mu), so DAG only flips the projector signs.
-template <int MU, int MODE, bool DAG, class SIO, class GIO>
+// NT: streaming link loads.
+template <int MU, int MODE, bool DAG, bool NT = false, class SIO, class GIO>
 __device__ __forceinline__ void hop_fwd(const SIO &in, const GIO &g, int p, int j, int jnb, typename SIO::C acc[12])
 {
    constexpr int SG = DAG ? 1 : -1;
@@ -364,13 +365,13 @@ __device__ __forceinline__ void hop_fwd(const SIO &in, const GIO &g, int p, int 
    typename GIO::U u;
    typename SIO::Hv r;
    in.load_sp(1 - p, jnb, f);
-   g.load_u(MODE == MODE_COMPAT ? 0 : p, MU, j, u);
+   g.template load_u<NT>(MODE == MODE_COMPAT ? 0 : p, MU, j, u);
    term_u<MU, SG>(f, u, r);
    accum<MU, SG, MODE != MODE_COMPAT>(acc, r);
 }
 
 // Backward term of direction MU; jnb = site of x-mu (its link U_mu(x-mu) too).
-template <int MU, bool DAG, class SIO, class GIO>
+template <int MU, bool DAG, bool NT = false, class SIO, class GIO>
 __device__ __forceinline__ void hop_bwd(const SIO &in, const GIO &g, int p, int jnb, typename SIO::C acc[12])
 {
    constexpr int SG = DAG ? -1 : 1;
@@ -378,17 +379,17 @@ __device__ __forceinline__ void hop_bwd(const SIO &in, const GIO &g, int p, int 
    typename GIO::U u;
    typename SIO::Hv r;
    in.load_sp(1 - p, jnb, f);
-   g.load_u(1 - p, MU, jnb, u);
+   g.template load_u<NT>(1 - p, MU, jnb, u);
    term_udag<MU, SG>(f, u, r);
    accum<MU, SG, true>(acc, r);
 }
 
-template <int MU, int MODE, bool DAG, class SIO, class GIO>
+template <int MU, int MODE, bool DAG, bool NT = false, class SIO, class GIO>
 __device__ __forceinline__ void hop_dir(const SIO &in, const GIO &g, int p, int j, const Nbr &n,
                                         typename SIO::C acc[12])
 {
-   hop_fwd<MU, MODE, DAG>(in, g, p, j, n.up[MU], acc);
-   hop_bwd<MU, DAG>(in, g, p, n.dn[MU], acc);
+   hop_fwd<MU, MODE, DAG, NT>(in, g, p, j, n.up[MU], acc);
+   hop_bwd<MU, DAG, NT>(in, g, p, n.dn[MU], acc);
 }
 
 // Maps the hardware block index to a logical tile.  Blocks are handed to
@@ -452,7 +453,7 @@ struct CgFuse {
 // registers, one wave per SIMD, against 144 and three waves).
 // EPI = 4 is EPI = 1 with the centre taken from another field, f.p: out =
 // c(x) - kappa_r * (H in)(x) (the even-odd operator's second half hop, whose
-// input lives on the other parity; gather kernel only).
+// input lives on the other parity; half-lattice kernel only).
 // With NORM the site's |out|^2 joins the deterministic chunk reduction.  `in`
 // and `out` are positioned at the RHS `r`, whose kappa and alpha apply.  `pre`,
 // when not null, is the site's spinor of b that EPI 3 reads, loaded earlier.
@@ -549,6 +550,48 @@ template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, class SIO, class GI
 __global__ __launch_bounds__(BLOCK) void hop_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> f)
 {
    hop_block<MODE, DAG, EPI, NORM, BLOCK>(in, out, g, a, logical_block(a), f);
+}
+
+// Half-lattice hop (eo or oe; EPI 0 or 4): the gather kernel's sites and order
+// of operations, in block orders and with link loads for one parity.
+//   It is bound by the bytes its L2s miss: each link is used once, and a
+// spinor by eight sites, so what the L2 holds should be spinors.  NT streams
+// the links past it; order 3 gives XCD k the k-th eighth of the column blocks
+// of a t-slice (a slab in z), swept through all t-slices, so that a spinor's t
+// neighbours find it in the L2 too.  us per half, F64: 32^3 x 64 364 -> 316
+// (NT; 1.6 GB compulsory, 5.1 TB/s), 28 x 20 x 36 x 44 152 -> 133 (NT), 24^3 x
+// 48 with 4 RHS 281 -> 256 (both), with 12 RHS 753 -> 648 (order 3).
+template <int MODE, int EPI, bool NT, int BLOCK, class SIO, class GIO>
+__global__ __launch_bounds__(BLOCK) void hop_half_kernel(SIO in, SIO out, GIO g, HopArgs a, CgFuse<SIO> f)
+{
+   typedef typename SIO::C C;
+   const int p = a.parity0;
+   const int r = threadIdx.x % a.R;
+   const int js = threadIdx.x / a.R;
+   const int rr = rhs_of(a, r);
+   int j, end;  // the lane's site; the first one past its block's t-slice (order 3) or the parity
+   if (a.order == 3) {
+      const int nbS = (a.S + a.spb - 1) / a.spb;
+      const int k = blockIdx.x & 7, i = blockIdx.x >> 3;
+      const int n = (nbS >> 3) + (k < (nbS & 7)), first = k * (nbS >> 3) + min(k, nbS & 7);
+      const int t = i / n;
+      j = t * a.S + (first + i - t * n) * a.spb + js;
+      end = t < a.L[3] ? (t + 1) * a.S : 0;
+   } else {
+      j = logical_block(a) * a.spb + js;
+      end = a.Vh;
+   }
+   if (js >= a.spb || j >= end) return;
+   const SIO si = in.at_rhs(rr);
+   const Nbr n = neighbours(a, p, j);
+   C acc[12];
+#pragma unroll
+   for (int c = 0; c < 12; c++) acc[c] = C{0, 0};
+   hop_dir<0, MODE, false, NT>(si, g, p, j, n, acc);
+   hop_dir<1, MODE, false, NT>(si, g, p, j, n, acc);
+   hop_dir<2, MODE, false, NT>(si, g, p, j, n, acc);
+   hop_dir<3, MODE, false, NT>(si, g, p, j, n, acc);
+   epilogue<EPI, false>(si, out.at_rhs(rr), a, rr, p, j, acc, (const C *)nullptr, f);
 }
 
 // RHS-blocked gather: each lane handles RB consecutive right-hand sides of
@@ -1401,7 +1444,7 @@ __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g,
 }
 
 // kernel variants: gather (1 RHS per lane), t-march, RHS-blocked gather, LDS tile, pipelined t-march
-enum Variant { V_GATHER = 0, V_MARCH = 1, V_RB2 = 2, V_RB4 = 4, V_TILE = 8, V_PIPE = 16 };
+enum Variant { V_GATHER = 0, V_MARCH = 1, V_RB2 = 2, V_RB4 = 4, V_TILE = 8, V_PIPE = 16, V_HALF = 32 };
 
 // S: the input field's accessor; SO: the output's (differs only with EPI 3,
 // which runs the gather kernel).  Returns 0 when the kernel was enqueued, and
@@ -1413,14 +1456,18 @@ int launch_one(int variant, dim3 grid, dim3 block, hipStream_t st, S si, SO so, 
                const CgFuse<S> &f)
 {
    constexpr bool same = std::is_same<S, SO>::value && EPI != 3;  // the tile and RHS-blocked kernels
-   if constexpr (EPI == 4) {  // the external-centre epilogue exists for the gather kernel only
-      if (variant == V_GATHER) {
-         hipLaunchKernelGGL((hop_kernel<MODE, DAG, EPI, NORM, BLOCK, S, G, SO>), grid, block, 0, st, si, so, gg, a, f);
+   if constexpr ((EPI == 0 || EPI == 4) && !DAG && !NORM && same) {
+      if (variant == V_HALF) {
+         if (a.stream_links)
+            hipLaunchKernelGGL((hop_half_kernel<MODE, EPI, true, BLOCK, S, G>), grid, block, 0, st, si, so, gg, a, f);
+         else
+            hipLaunchKernelGGL((hop_half_kernel<MODE, EPI, false, BLOCK, S, G>), grid, block, 0, st, si, so, gg, a, f);
          return 0;
       }
-      return plqcd::set_error(2, "hop: the external-centre epilogue runs the gather kernel only (variant %d)", variant);
    }
-   if (variant == V_PIPE) {
+   if constexpr (EPI == 4) {  // the external-centre epilogue exists for the half-lattice kernel only
+      return plqcd::set_error(2, "hop: the external-centre epilogue runs on one parity only (variant %d)", variant);
+   } else if (variant == V_PIPE) {
       if constexpr (BLOCK == 256) {
          const size_t lds = pipe_lds_bytes<MODE, G>(a.spb);
          if (links_per_slice<MODE>() * a.spb <= (int)block.x)
@@ -1480,7 +1527,7 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
    const S si = spinor_io<PREC>(in);
    const G gg = gauge_io<PREC, LINKS>(g);
    const bool resid = op.resid_b != nullptr;  // EPI 3: out may have another precision
-   const bool centre = op.centre != nullptr;  // EPI 4: the gather kernel only
+   const bool centre = op.centre != nullptr;  // EPI 4: one parity only
    // lanes: the window of right-hand sides [op.r0, op.r0 + R) of the fields
    const int R = op.nr > 0 ? op.nr : in->nrhs;
    a.r0 = op.nr > 0 && !op.rlist ? op.r0 : 0;
@@ -1491,7 +1538,7 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
                                        solver ? plqcd::kTuneOpSolver : plqcd::kTuneOpHop},
                         &tu);
    // RHS per lane (RHS-blocked gather) when it divides R; none for the
-   // residual epilogue, and the external-centre one runs the gather kernel only
+   // residual epilogue, and the external-centre one runs the half-lattice kernel only
    const int rb = !resid && !centre && (tu.rb == 2 || tu.rb == 4) && R % tu.rb == 0 ? tu.rb : 1;
    const int lanes = R / rb;  // lanes per site
    // block shape: `lanes` lanes per site and a whole number of reduction chunks
@@ -1542,7 +1589,8 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
                       (!norm || (lat->Lxh * tu.ty) % REDUCE_CHUNK == 0);
    // the pipelined t-march wherever it fits (four right-hand sides or more)
    const bool pipe = march && !tiled && pipe_fits<G>(mode, a.spb, threads);
-   const int variant = tiled ? V_TILE : pipe ? V_PIPE : march ? V_MARCH : (rb == 2 ? V_RB2 : rb == 4 ? V_RB4 : V_GATHER);
+   const bool half = a.nparity == 1 && !dag && !norm && rb == 1 && (epi == 0 || epi == 4);
+   const int variant = half ? V_HALF : tiled ? V_TILE : pipe ? V_PIPE : march ? V_MARCH : (rb == 2 ? V_RB2 : rb == 4 ? V_RB4 : V_GATHER);
    a.nt = march ? (lat->L[3] + tu.tmarch - 1) / tu.tmarch : 1;
    int nb, nthreads = threads, mblock = pipe ? 256 : maxblock;
    if (tiled) {
@@ -1560,6 +1608,28 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
    if (pipe && tu.gy > 0 && lat->Lxh * lat->L[1] % (a.spb * tu.gy) == 0 && lat->L[2] % tu.gz == 0) {
       a.gy = tu.gy;
       a.gz = tu.gz;
+   }
+   if (half) {
+      // Links stream past the L2s unless the field of links about fits them (32
+      // MB together) and is there from the last call, or many RHS share each
+      // load: one RHS, us per half without and with, F32 12-real 16^3 x 32 (25
+      // MB of links) 8.7 and 10.7, 20^3 x 40 (61 MB) 18.1 and 22.0, 24^3 x 48
+      // (127 MB) 42.9 and 40.5; F64 16^3 x 32 (75 MB) 21.2 and 21.4, 20^3 x 40
+      // (184 MB) 56.7 and 48.8; F64 24^3 x 48 4 RHS 281 and 268, 6 RHS 392 and
+      // 386, 12 RHS 753 and 780.
+      a.stream_links = R <= 4 && g->bytes >= size_t(75) << 20;
+      // Slabs where t-slices of several RHS crowd each other out: without and
+      // with, F64 24^3 x 48 with 4 RHS (a field of 510 MB) 268 and 256, 16^3 x 32
+      // with 4 RHS (101 MB) 54 and 59, with 12 RHS (302 MB) 150 and 145; one RHS
+      // at 32^3 x 64 (403 MB) 316 and 341.
+      HopTuning user{};
+      if (!plqcd::user_tuning(PREC, &user)) {
+         const int nbS = (a.S + a.spb - 1) / a.spb, most = (nbS + 7) / 8;
+         const bool slab = R >= 4 && in->bytes * (double(R) / in->nrhs) >= double(size_t(200) << 20) &&
+                           8 * most <= nbS + nbS / 8;  // an XCD's slab at most an eighth larger than the mean
+         a.order = slab ? 3 : 1;
+         if (slab) nb = 8 * most * lat->L[3];
+      }
    }
    const dim3 grid(nb), block(nthreads);
    hipStream_t st = lat->stream;

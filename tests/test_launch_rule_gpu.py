@@ -104,3 +104,33 @@ def test_batch_of_small_ragged_lattices(hp):
         for s, w in zip(sets, want):
             for r in range(s[3].nrhs):
                 assert np.array_equal(s[3].download(r), w[r]), (s[0].L, mode, r)
+
+
+# smallest lattices on which a half-lattice launch streams its links (a gauge
+# field of 75 MiB) and sweeps slabs (200 MiB of the input), and one below both
+@pytest.mark.parametrize("L,prec,links,R", [((16, 16, 18, 32), 0, 18, 1), ((16, 16, 18, 32), 0, 18, 4),
+                                            ((12, 18, 10, 22), 0, 12, 12), ((20, 16, 18, 32), 1, 18, 12),
+                                            ((4, 6, 6, 4), 2, 12, 5)])
+def test_half_lattice_orders(hp, L, prec, links, R):
+    """The built-in rule's orders and link loads give bitwise the plain order's
+    output, on each parity, and leave the other alone."""
+    lat, g, fi, fo, qs, u = fields(hp, L, prec, links, R)
+    mark = np.full_like(qs[0], 3.0)
+    half = len(mark) // 2
+    try:
+        for mode, parity in ((hp.HOP_WILSON, 0), (hp.HOP_COMPAT, 1)):
+            mine = slice(parity * half, (parity + 1) * half)
+            other = slice((1 - parity) * half, (2 - parity) * half)
+            got = []
+            for shape in ((0, 1, 256, 0, 1, 0, 0), None):
+                set_shape(prec, shape)
+                for r in range(R):
+                    fo.upload(mark, r)
+                hp.hop(g, fi, fo, parity, mode)
+                got.append([fo.download(r) for r in range(R)])
+            for want, out in zip(*got):
+                assert np.array_equal(out[mine], want[mine])
+                assert np.array_equal(out[other], mark[other])
+                assert not np.array_equal(out[mine], mark[mine])
+    finally:
+        set_shape(prec, None)
