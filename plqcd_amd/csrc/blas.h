@@ -15,6 +15,17 @@ struct Window {
 
 size_t partial_doubles(const plqcd_hip_field *f);
 
+// Per-RHS scalars of a CG iteration (device arrays); count: zeros between
+// launches.
+struct CgScalars {
+   double *rr, *rr_new, *rr_prev, *pap, *alpha, *beta;
+   const int *active;
+   unsigned *count;
+};
+// Sums the chunks of RHS 0 .. R-1 as reduce_partials does and forms the scalar
+// that follows: op 0 pap and alpha, op 1 rr_new and beta (and rr moves on).
+int reduce_cg(int op, double *partial, size_t stride, int n, int R, const CgScalars &c, hipStream_t st);
+
 // x += alpha p in the working precision of the storage (float for F32/F16,
 // double for F64), then p = r + beta p in double, from one read of p
 int blas_cg_step(const plqcd_hip_field *r, const double *beta, plqcd_hip_field *p, const double *alpha,

@@ -94,8 +94,8 @@ class CgEngine {
    plqcd_hip_field *t1_ = nullptr;                                                  // F64
    plqcd_hip_field *rs_ = nullptr, *ps_ = nullptr, *qs_ = nullptr, *xs_ = nullptr;  // sloppy
    double *partial_ = nullptr;
-   double *scal_ = nullptr;  // kappa, rr, rr_new, pap, alpha, beta, tmp (7 x S)
-   int *imask_ = nullptr;    // active, update, the list of slots being updated (3 x S)
+   double *scal_ = nullptr;  // kappa, rr, rr_new, pap, alpha, beta, tmp, rr_prev (8 x S)
+   int *imask_ = nullptr;    // active, update, the list of slots being updated, the reductions' counters (4 x S)
    double *host_ = nullptr;  // pinned: rr_new, tmp (2 x S)
    int *hmask_ = nullptr;    // pinned: active, update, update list (3 x S), the sources of their uploads
    hipEvent_t ev_ = nullptr; // recorded after each enqueued iteration / reliable update
@@ -114,9 +114,15 @@ class CgEngine {
    double *alpha_d() { return scal_ + 4 * S_; }
    double *beta_d() { return scal_ + 5 * S_; }
    double *tmp_d() { return scal_ + 6 * S_; }
+   double *rr_prev_d() { return scal_ + 7 * S_; }
    int *active_d() { return imask_; }
    int *update_d() { return imask_ + S_; }
    int *ulist_d() { return imask_ + 2 * S_; }
+   CgScalars scalars()
+   {
+      return CgScalars{rr_d(),    rr_new_d(), rr_prev_d(), pap_d(),
+                       alpha_d(), beta_d(),   active_d(),  reinterpret_cast<unsigned *>(imask_ + 3 * S_)};
+   }
 };
 
 }  // namespace plqcd

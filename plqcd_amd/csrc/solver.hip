@@ -11,11 +11,11 @@
 // replaces the iterated one.  A slot stops when its FP64 true residual meets
 // its tolerance.
 //
-// One iteration is a fixed sequence of kernels whose scalars live on the
-// device: beta; one pass that applies the previous iteration's x += alpha p
-// and forms p = r + beta p; M p with |Mp|^2; alpha; then M^+ (Mp) with the
+// One iteration is a fixed sequence of five kernels whose scalars live on the
+// device: one pass that applies the previous iteration's x += alpha p and forms
+// p = r + beta p; M p with |Mp|^2; the sum and alpha; then M^+ (Mp) with the
 // residual update r -= alpha Ap and |r|^2 fused into its epilogue, so Ap is
-// never stored.  The iterate therefore trails by one step: a reliable update
+// never stored; the sum and the next beta.  The iterate therefore trails by one step: a reliable update
 // first applies the pending x += alpha p of the slots it updates and zeroes
 // their alpha, so the next pass adds nothing twice.  The arithmetic of each
 // update is unchanged, and so are the iterates.  The sequence is captured
@@ -36,29 +36,27 @@ namespace {
 
 constexpr int kMaxSlots = 32;
 
-__global__ void k_alpha(const double *rr, const double *pap, const int *active, double *alpha, int S)
-{
-   const int r = threadIdx.x;
-   if (r < S) alpha[r] = (active[r] && pap[r] > 0.0) ? rr[r] / pap[r] : 0.0;
-}
-
-__global__ void k_beta(double *rr, const double *rr_new, const int *active, double *beta, int S)
+// The next iteration's beta = rr_new / rr again, after reliable updates have
+// changed rr_new and the active slots (the iteration's reduction has formed it
+// from the iterated residual and kept the rr it used in rr_prev).
+__global__ void k_beta(const plqcd::CgScalars c, int S)
 {
    const int r = threadIdx.x;
    if (r < S) {
-      beta[r] = (active[r] && rr[r] > 0.0) ? rr_new[r] / rr[r] : 0.0;
-      rr[r] = rr_new[r];
+      c.beta[r] = (c.active[r] && c.rr_prev[r] > 0.0) ? c.rr_new[r] / c.rr_prev[r] : 0.0;
+      c.rr[r] = c.rr_new[r];
    }
 }
 
-// rr[s] = rr_new[s] = src[s] and alpha[s] = 0 (no pending iterate update)
-// for the slots in mask
-__global__ void k_admit(const int *mask, const double *src, double *rr, double *rr_new, double *alpha, int S)
+// rr[s] = rr_new[s] = rr_prev[s] = src[s], beta[s] = rr_new / rr (p is zero)
+// and alpha[s] = 0 (no pending iterate update) for the slots in mask
+__global__ void k_admit(const int *mask, const double *src, const plqcd::CgScalars c, int S)
 {
    const int r = threadIdx.x;
    if (r < S && mask[r]) {
-      rr[r] = rr_new[r] = src[r];
-      alpha[r] = 0.0;
+      c.rr[r] = c.rr_new[r] = c.rr_prev[r] = src[r];
+      c.beta[r] = src[r] > 0.0 ? src[r] / src[r] : 0.0;
+      c.alpha[r] = 0.0;
    }
 }
 
@@ -143,15 +141,15 @@ int CgEngine::alloc(int sloppy)
       if (int rc = plqcd_hip_field_create(lat_, PLQCD_PREC_F64, S_, &t1_)) return rc;
    }
    PLQCD_HIP_TRY(hipMalloc(&partial_, partial_doubles(b_) * sizeof(double)));
-   PLQCD_HIP_TRY(hipMalloc(&scal_, 7 * S_ * sizeof(double)));
-   PLQCD_HIP_TRY(hipMalloc(&imask_, 3 * S_ * sizeof(int)));
+   PLQCD_HIP_TRY(hipMalloc(&scal_, 8 * S_ * sizeof(double)));
+   PLQCD_HIP_TRY(hipMalloc(&imask_, 4 * S_ * sizeof(int)));
    PLQCD_HIP_TRY(hipHostMalloc(&host_, 2 * S_ * sizeof(double), hipHostMallocDefault));
    PLQCD_HIP_TRY(hipHostMalloc(&hmask_, 3 * S_ * sizeof(int), hipHostMallocDefault));
    PLQCD_HIP_TRY(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
    hipStream_t st = lat_->stream;
-   std::vector<double> z(7 * S_, 0.0);
+   std::vector<double> z(8 * S_, 0.0);
    PLQCD_HIP_TRY(hipMemcpyAsync(scal_, z.data(), z.size() * sizeof(double), hipMemcpyHostToDevice, st));
-   std::vector<int> zi(3 * S_, 0);
+   std::vector<int> zi(4 * S_, 0);
    PLQCD_HIP_TRY(hipMemcpyAsync(imask_, zi.data(), zi.size() * sizeof(int), hipMemcpyHostToDevice, st));
    if (int rc = blas_zero(ps_, nullptr)) return rc;
    if (int rc = blas_zero(xs_, nullptr)) return rc;
@@ -220,8 +218,7 @@ int CgEngine::admit(const std::vector<int> &which, const double *kappa, const do
    if (int rc = blas_zero(ps_, update_d(), w)) return rc;
    if (int rc = blas_copy(rs_, b_, partial_, update_d(), w)) return rc;
    if (int rc = reduce_partials(partial_, 2 * nc, 0, 2 * nc, w.nr, tmp_d(), st, w.r0)) return rc;
-   hipLaunchKernelGGL(k_admit, dim3(1), dim3(kMaxSlots), 0, st, update_d(), tmp_d(), rr_d(), rr_new_d(), alpha_d(),
-                      S_);
+   hipLaunchKernelGGL(k_admit, dim3(1), dim3(kMaxSlots), 0, st, update_d(), tmp_d(), scalars(), S_);
    PLQCD_HIP_TRY(hipGetLastError());
    PLQCD_HIP_TRY(hipMemcpyAsync(host_ + S_, tmp_d(), S_ * sizeof(double), hipMemcpyDeviceToHost, st));
    PLQCD_HIP_TRY(hipStreamSynchronize(st));
@@ -267,7 +264,6 @@ int CgEngine::iteration(int nr)
    hipStream_t st = lat_->stream;
    const int nc = reduce_chunks(lat_->Vh);
    const Window w{0, nr};
-   hipLaunchKernelGGL(k_beta, dim3(1), dim3(kMaxSlots), 0, st, rr_d(), rr_new_d(), active_d(), beta_d(), S_);
    // xs += alpha ps (alpha of the last iteration), then ps = rs + beta ps
    if (int rc = blas_cg_step(rs_, beta_d(), ps_, alpha_d(), xs_, w)) return rc;
    DslashOp m;
@@ -275,8 +271,7 @@ int CgEngine::iteration(int nr)
    m.kappa = kappa_d();
    m.partial = partial_;
    if (int rc = dslash(gs_, ps_, qs_, PLQCD_PARITY_ALL, PLQCD_HOP_WILSON, m)) return rc;
-   if (int rc = reduce_partials(partial_, 2 * nc, 0, 2 * nc, nr, pap_d(), st)) return rc;
-   hipLaunchKernelGGL(k_alpha, dim3(1), dim3(kMaxSlots), 0, st, rr_d(), pap_d(), active_d(), alpha_d(), S_);
+   if (int rc = reduce_cg(0, partial_, 2 * nc, 2 * nc, nr, scalars(), st)) return rc;
    // Ap = M^+ q, fused with rs -= alpha Ap and |rs|^2
    DslashOp md;
    md.nr = nr;
@@ -285,7 +280,7 @@ int CgEngine::iteration(int nr)
    md.partial = partial_;
    md.alpha = alpha_d();
    if (int rc = dslash(gs_, qs_, rs_, PLQCD_PARITY_ALL, PLQCD_HOP_WILSON, md)) return rc;
-   if (int rc = reduce_partials(partial_, 2 * nc, 0, 2 * nc, nr, rr_new_d(), st)) return rc;
+   if (int rc = reduce_cg(1, partial_, 2 * nc, 2 * nc, nr, scalars(), st)) return rc;
    PLQCD_HIP_TRY(hipGetLastError());
    return 0;
 }
@@ -454,6 +449,8 @@ int CgEngine::end_finish(std::vector<int> &finished)
    std::copy(active_.begin(), active_.end(), hmask_);
    PLQCD_HIP_TRY(hipMemcpyAsync(rr_new_d(), host_, S_ * sizeof(double), hipMemcpyHostToDevice, st));
    PLQCD_HIP_TRY(hipMemcpyAsync(active_d(), hmask_, S_ * sizeof(int), hipMemcpyHostToDevice, st));
+   hipLaunchKernelGGL(k_beta, dim3(1), dim3(kMaxSlots), 0, st, scalars(), S_);
+   PLQCD_HIP_TRY(hipGetLastError());
    return 0;
 }
 
