@@ -16,20 +16,29 @@ struct Window {
 size_t partial_doubles(const plqcd_hip_field *f);
 
 // Per-RHS scalars of a CG iteration (device arrays); count: zeros between
-// launches.
+// launches; thr: the residual norm at which the host has to look at a RHS.
+//
+// Several iterations may be enqueued before the host looks.  halt[0] tells an
+// iteration's kernels to do nothing, halt[1] the next iteration's: the first
+// kernel (blas_cg_step) sets halt[1] = halt[0], and the last (op 1) sets it when
+// an active RHS has come down to its threshold or is no longer finite.
 struct CgScalars {
    double *rr, *rr_new, *rr_prev, *pap, *alpha, *beta;
+   const double *thr;
    const int *active;
    unsigned *count;
+   int *halt;
 };
 // Sums the chunks of RHS 0 .. R-1 as reduce_partials does and forms the scalar
-// that follows: op 0 pap and alpha, op 1 rr_new and beta (and rr moves on).
+// that follows: op 0 pap and alpha, op 1 rr_new and beta (and rr moves on) and
+// halt[1].
 int reduce_cg(int op, double *partial, size_t stride, int n, int R, const CgScalars &c, hipStream_t st);
 
 // x += alpha p in the working precision of the storage (float for F32/F16,
-// double for F64), then p = r + beta p in double, from one read of p
-int blas_cg_step(const plqcd_hip_field *r, const double *beta, plqcd_hip_field *p, const double *alpha,
-                 plqcd_hip_field *x, const Window &w = Window{});
+// double for F64), then p = r + beta p in double, from one read of p (alpha,
+// beta and halt of `c`)
+int blas_cg_step(const plqcd_hip_field *r, plqcd_hip_field *p, plqcd_hip_field *x, const CgScalars &c,
+                 const Window &w = Window{});
 // x += alpha p as in blas_cg_step, for the RHS with mask[r] != 0 only (mask required)
 int blas_x_step(const double *alpha, const plqcd_hip_field *p, plqcd_hip_field *x, const int *mask,
                 const Window &w = Window{});

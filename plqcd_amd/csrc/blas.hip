@@ -56,9 +56,13 @@ __device__ __forceinline__ void x_step(const SpinorIO<P> &X, const typename Spin
 // read of p: the iterate update of the last CG iteration, deferred to this
 // pass, and the new search direction
 template <int P>
-__global__ __launch_bounds__(kBlock) void k_cg_step(SpinorIO<P> rv, const double *beta, SpinorIO<P> pv,
-                                                    const double *alpha, SpinorIO<P> xv, BlasArgs a)
+__global__ __launch_bounds__(kBlock) void k_cg_step(SpinorIO<P> rv, SpinorIO<P> pv, SpinorIO<P> xv,
+                                                    plqcd::CgScalars cs, BlasArgs a)
 {
+   const double *alpha = cs.alpha, *beta = cs.beta;
+   const int halted = cs.halt[0];
+   if (blockIdx.x == 0 && threadIdx.x == 0) cs.halt[1] = halted;
+   if (halted) return;
    int p, j, js, r;
    if (!blas_site(a, p, j, js, r)) return;
    const SpinorIO<P> Rr = rv.at_rhs(r), Pp = pv.at_rhs(r);
@@ -194,6 +198,7 @@ __global__ __launch_bounds__(256) void k_reduce_cg(double *partial, size_t strid
 {
    __shared__ bool last;
    const int b = blockIdx.x, nseg = gridDim.x, r = blockIdx.y, t = threadIdx.x;
+   if (c.halt[0]) return;
    double *base = partial + r * stride, *p = base + (size_t)b * kSeg;
    const int m = min(kSeg, n - b * kSeg);
    double s = 0.0;
@@ -220,6 +225,8 @@ __global__ __launch_bounds__(256) void k_reduce_cg(double *partial, size_t strid
       c.beta[r] = (c.active[r] && rr > 0.0) ? sum / rr : 0.0;
       c.rr_prev[r] = rr;
       c.rr[r] = sum;
+      if (c.active[r] && (!(sqrt(sum) > c.thr[r]) || !isfinite(sum)))
+         __hip_atomic_store(c.halt + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
    }
 }
 
@@ -295,8 +302,8 @@ int reduce_cg(int op, double *partial, size_t stride, int n, int R, const CgScal
 
 size_t partial_doubles(const plqcd_hip_field *f) { return (size_t)f->nrhs * 2 * reduce_chunks(f->lat->Vh); }
 
-int blas_cg_step(const plqcd_hip_field *r, const double *beta, plqcd_hip_field *p, const double *alpha,
-                 plqcd_hip_field *x, const Window &w)
+int blas_cg_step(const plqcd_hip_field *r, plqcd_hip_field *p, plqcd_hip_field *x, const CgScalars &c,
+                 const Window &w)
 {
    if (int rc = check_pair(r, p, w) | check_pair(r, x, w)) return rc;
    if (r->prec != p->prec || r->prec != x->prec) return set_error(1, "blas_cg_step: precision mismatch");
@@ -305,8 +312,8 @@ int blas_cg_step(const plqcd_hip_field *r, const double *beta, plqcd_hip_field *
    hipStream_t st = r->lat->stream;
    return dispatch1(r->prec, [&](auto P) {
       constexpr int PP = decltype(P)::value;
-      hipLaunchKernelGGL(k_cg_step<PP>, grid_of(a), block_of(a), 0, st, spinor_io<PP>(r), beta, spinor_io<PP>(p),
-                         alpha, spinor_io<PP>(x), a);
+      hipLaunchKernelGGL(k_cg_step<PP>, grid_of(a), block_of(a), 0, st, spinor_io<PP>(r), spinor_io<PP>(p),
+                         spinor_io<PP>(x), c, a);
    });
 }
 

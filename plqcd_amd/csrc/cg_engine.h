@@ -50,10 +50,13 @@ class CgEngine {
    // Uploads host sources into the listed slots and admits them together.
    int admit_host(const std::vector<int> &which, const std::vector<const spinor *> &b_host, double kappa, double tol,
                   int max_iter);
-   // Enqueues one iteration of all active slots (asynchronous).  The kernels
-   // cover the slots up to the highest active one; each such width has its
-   // own captured graph.
-   int launch();
+   // Enqueues one iteration of all active slots, or up to `ahead` of them
+   // (asynchronous).  The kernels cover the slots up to the highest active one;
+   // each such width has its own captured graph.  Of several iterations those
+   // after the first that brings a slot to a reliable update do nothing (the
+   // device decides it by a threshold no tighter than the host's rule), so the
+   // iterates are those of one iteration at a time.
+   int launch(int ahead = 1);
    // Waits for the iteration, runs the reliable updates it calls for and
    // appends the slots that finished to `finished`.
    int finish(std::vector<int> &finished);
@@ -80,9 +83,11 @@ class CgEngine {
   private:
    CgEngine() = default;
    int alloc(int sloppy);
-   int iteration(int nr);
+   int iteration(int nr, int j);
+   int iterations(int nr, int n);
    int reliable_update();
-   int capture(int nr);
+   int capture(int nr, int n);
+   int upload_thresholds();
 
    plqcd_hip_lattice *lat_ = nullptr;
    const plqcd_hip_gauge *g_ = nullptr, *gs_ = nullptr;
@@ -94,34 +99,42 @@ class CgEngine {
    plqcd_hip_field *t1_ = nullptr;                                                  // F64
    plqcd_hip_field *rs_ = nullptr, *ps_ = nullptr, *qs_ = nullptr, *xs_ = nullptr;  // sloppy
    double *partial_ = nullptr;
-   double *scal_ = nullptr;  // kappa, rr, rr_new, pap, alpha, beta, tmp, rr_prev (8 x S)
+   // kappa, rr, thr, pap, alpha, beta, tmp, rr_prev, rr_new (9 x S), and the halt flags (kFlags ints)
+   double *scal_ = nullptr;
    int *imask_ = nullptr;    // active, update, the list of slots being updated, the reductions' counters (4 x S)
-   double *host_ = nullptr;  // pinned: rr_new, tmp (2 x S)
+   double *host_ = nullptr;  // pinned: rr_new and the halt flags as on the device, tmp, thr
+   int launched_ = 0;        // iterations of the last launch
    int *hmask_ = nullptr;    // pinned: active, update, update list (3 x S), the sources of their uploads
    hipEvent_t ev_ = nullptr; // recorded after each enqueued iteration / reliable update
    struct Graph {
       hipGraph_t def = nullptr;
       hipGraphExec_t exec = nullptr;
    };
-   std::vector<Graph> graphs_;  // by window width 1..S
+   static constexpr int kMostAhead = 4, kFlags = 2 * ((kMostAhead + 2) / 2);  // iterations per launch; their flags, in pairs
+   std::vector<Graph> graphs_[kMostAhead + 1];  // by iterations, by window width 1..S
    std::vector<CgSlot> slot_;
    std::vector<int> active_, update_;
 
    double *kappa_d() { return scal_; }
    double *rr_d() { return scal_ + S_; }
-   double *rr_new_d() { return scal_ + 2 * S_; }
+   double *thr_d() { return scal_ + 2 * S_; }
    double *pap_d() { return scal_ + 3 * S_; }
    double *alpha_d() { return scal_ + 4 * S_; }
    double *beta_d() { return scal_ + 5 * S_; }
    double *tmp_d() { return scal_ + 6 * S_; }
    double *rr_prev_d() { return scal_ + 7 * S_; }
+   double *rr_new_d() { return scal_ + 8 * S_; }
+   int *halt_d() { return reinterpret_cast<int *>(scal_ + 9 * S_); }
+   const int *host_halt() const { return reinterpret_cast<const int *>(host_ + S_); }
+   double *host_tmp() { return host_ + S_ + kFlags / 2; }
+   double *host_thr() { return host_tmp() + S_; }
    int *active_d() { return imask_; }
    int *update_d() { return imask_ + S_; }
    int *ulist_d() { return imask_ + 2 * S_; }
-   CgScalars scalars()
+   CgScalars scalars(int j = 0)  // of the j-th iteration of a launch
    {
-      return CgScalars{rr_d(),    rr_new_d(), rr_prev_d(), pap_d(),
-                       alpha_d(), beta_d(),   active_d(),  reinterpret_cast<unsigned *>(imask_ + 3 * S_)};
+      return CgScalars{rr_d(),  rr_new_d(), rr_prev_d(), pap_d(), alpha_d(),
+                       beta_d(), thr_d(),   active_d(),  reinterpret_cast<unsigned *>(imask_ + 3 * S_), halt_d() + j};
    }
 };
 

@@ -24,6 +24,7 @@ struct HopArgs {
    int nchunk;   // reduction chunks per parity
    const double *kappa;  // per-RHS kappa of M = 1 - kappa H (EPI = 1)
    double *partial;      // [R][2*nchunk] chunk sums of |out|^2 (NORM)
+   const int *halt;      // NORM launches: do nothing when set and not zero (null: never)
 };
 
 // Launch shape of the hopping kernels, process-wide.
@@ -65,6 +66,8 @@ namespace plqcd {
 //                    out = resid_b - (in - kappa H^+ in) for every RHS of the
 //                    launch, stored in out's own precision (any), and its |out|^2
 //                    to partial
+//   halt    != null: (with partial) the launch does nothing when *halt, a device
+//                    flag, is not zero
 //   nr      > 0:     only the right-hand sides r0 .. r0+nr-1 of the fields (kappa,
 //                    alpha and partial stay indexed by the field's RHS)
 //   rlist   != null: only the nr right-hand sides rlist[0 .. nr-1] (a device
@@ -78,6 +81,7 @@ struct DslashOp {
    const double *alpha = nullptr;
    const plqcd_hip_field *centre = nullptr;
    const plqcd_hip_field *resid_b = nullptr;
+   const int *halt = nullptr;
 };
 
 int dslash(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_field *out, int parity, int mode,

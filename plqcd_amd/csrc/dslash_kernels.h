@@ -549,6 +549,7 @@ __device__ __forceinline__ void hop_block(const SIO &in, const SO &out, const GI
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, class SIO, class GIO, class SO>
 __global__ __launch_bounds__(BLOCK) void hop_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> f)
 {
+   if (NORM && a.halt && *a.halt) return;
    hop_block<MODE, DAG, EPI, NORM, BLOCK>(in, out, g, a, logical_block(a), f);
 }
 
@@ -671,6 +672,7 @@ __device__ __forceinline__ void hop_block_rb(const SIO &in, const SIO &out, cons
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, int RB, class SIO, class GIO>
 __global__ __launch_bounds__(BLOCK) void hop_rb_kernel(SIO in, SIO out, GIO g, HopArgs a, CgFuse<SIO> f)
 {
+   if (NORM && a.halt && *a.halt) return;
    hop_block_rb<MODE, DAG, EPI, NORM, BLOCK, RB>(in, out, g, a, logical_block(a), f);
 }
 
@@ -876,6 +878,7 @@ __device__ __forceinline__ void hop_tmarch_block(const SIO &in, const SO &out, c
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, class SIO, class GIO, class SO>
 __global__ __launch_bounds__(BLOCK) void hop_tmarch_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
 {
+   if (NORM && a.halt && *a.halt) return;
    hop_tmarch_block<MODE, DAG, EPI, NORM, BLOCK>(in, out, g, a, logical_block(a), fuse);
 }
 
@@ -1165,6 +1168,7 @@ constexpr int pipe_waves()
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, int NIT, class SIO, class GIO, class SO>
 __global__ __launch_bounds__(BLOCK, pipe_waves<SIO>()) void hop_pipe_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
 {
+   if (NORM && a.halt && *a.halt) return;
    hop_pipe_block<MODE, DAG, EPI, NORM, BLOCK, NIT>(in, out, g, a, logical_block(a), fuse);
 }
 
@@ -1293,6 +1297,7 @@ __device__ __forceinline__ void tile_dir(const SIO &in, const GIO &g, const type
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, class SIO, class GIO>
 __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
 {
+   if (NORM && a.halt && *a.halt) return;
    typedef typename SIO::C C;
    const int r0 = rhs_of(a, 0);  // the launch's one RHS
    in = in.at_rhs(r0);
@@ -1555,6 +1560,7 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
    const int maxblock = threads <= 128 ? 128 : threads <= 256 ? 256 : 512;
    a.kappa = op.kappa;
    a.partial = op.partial;
+   a.halt = op.halt;
    a.nchunk = plqcd::reduce_chunks(lat->Vh);
    const bool dag = op.dag != 0;
    const int epi = resid ? 3 : op.alpha ? 2 : op.centre ? 4 : op.kappa ? 1 : 0;

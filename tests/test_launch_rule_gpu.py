@@ -134,3 +134,29 @@ def test_half_lattice_orders(hp, L, prec, links, R):
                 assert not np.array_equal(out[mine], mark[mine])
     finally:
         set_shape(prec, None)
+
+
+@pytest.mark.parametrize("prec,links", [(0, 18), (2, 12)])
+def test_iterations_enqueued_ahead(hp, prec, links):
+    """Solves stopped after 1 .. 9 iterations (whole and broken groups of four,
+    updates inside and at the end of one) take the iterates that direct
+    launches without graphs take; the iteration count is exact."""
+    from plqcd_amd import solver
+    L = (4, 6, 4, 10)
+    lat, g, b, x, qs, u = fields(hp, L, hp.PREC_F64, 18, 3)
+    gs = None if prec == hp.PREC_F64 else hp.Gauge(lat, prec, links).upload(u)
+    x2 = hp.Field(lat, hp.PREC_F64, 3)
+    tol = [1e-10, 1e-3, 1e-6]  # slots that stop at different iterations
+    for most in (1, 2, 3, 4, 5, 7, 8, 9, 200):
+        st = solver.cg_solve(g, b, x, 0.12, tol, max_iter=most, sloppy=gs)
+        st2 = solver.cg_solve(g, b, x2, 0.12, tol, max_iter=most, sloppy=gs, use_graph=False)
+        for r in range(3):
+            assert st[r]["iterations"] <= most
+            assert st[r]["converged"] or st[r]["iterations"] == most
+            assert st[r]["iterations"] == st2[r]["iterations"]
+            assert np.array_equal(x.download(r), x2.download(r))
+            # alone, the slot takes the same iterates
+            b1, x1 = hp.Field(lat).upload(qs[r]), hp.Field(lat)
+            s1 = solver.cg_solve(g, b1, x1, 0.12, tol[r], max_iter=most, sloppy=gs)[0]
+            assert s1["iterations"] == st[r]["iterations"]
+            assert np.array_equal(x1.download(), x.download(r))
