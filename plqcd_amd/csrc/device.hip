@@ -371,8 +371,15 @@ extern "C" size_t plqcd_hip_gauge_bytes(const plqcd_hip_gauge *g) { return g ? g
 extern "C" int plqcd_hip_gauge_upload(plqcd_hip_gauge *g, const su3 *u)
 {
    if (!g || !u) return plqcd::set_error(1, "plqcd_hip_gauge_upload: null argument");
+   return plqcd::gauge_upload_range(g, u, 0, g->lat->V);
+}
+
+int plqcd::gauge_upload_range(plqcd_hip_gauge *g, const su3 *u, int first, int last)
+{
    plqcd_hip_lattice *lat = g->lat;
-   return upload_chunks(lat, u, sizeof(su3), 0, size_t(4) * lat->V, [&](void *d, size_t l0, size_t n) {
+   if (first < 0 || last > lat->V || first > last) return plqcd::set_error(1, "bad site range");
+   return upload_chunks(lat, u, sizeof(su3), size_t(4) * first, size_t(4) * (last - first),
+                        [&](void *d, size_t l0, size_t n) {
       hipLaunchKernelGGL(pack_gauge, dim3((unsigned)((n + kPackBlock - 1) / kPackBlock)), dim3(kPackBlock), 0,
                          lat->stream, static_cast<const d2 *>(d), g->data, g->prec, g->links, lat->Vh, (int)l0,
                          (int)n);

