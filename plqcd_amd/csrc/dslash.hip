@@ -27,11 +27,12 @@
 // blocks no longer run faster for being fewer (latency), k the kernel's time
 // per lane and slice relative to the others, `waves` how many waves of it a
 // SIMD's registers hold.  The gather kernel has no chunks and no rounds to
-// speak of.  The constants were fitted to timings of every shape of 8 lattices
-// from 8^3 x 16 to 32^3 x 64, 28 x 20 x 36 x 44 and 34 x 22 x 30 x 30 among
-// them, with one RHS, and of 6 lattices with 4 and 12 RHS; the shapes they
-// pick take on average 0-1.4 % (F64), 1-3 % (F32) and 1-3 % (F16) longer than
-// the fastest one timed, 16 % at most.
+// speak of.  The constants were fitted to timings of every shape of 14 lattices
+// from 8^3 x 16 to 32^3 x 64, ten of them with extents that are no powers of
+// two (28 x 20 x 36 x 44, 32 x 42 x 24 x 64, 10 x 16 x 14 x 54 and so on), with
+// 1, 2 and 3 RHS, and of 6 lattices with 4 and 12 RHS.  The shapes they pick take
+// on average 3 to 6 % longer than the fastest one timed, depending on the
+// format, and 17 % at most.
 namespace {
 constexpr int kCus = 256;
 constexpr int kPipeRhs = 4;  // right-hand sides from which the pipelined t-march runs (pipe_fits)
@@ -46,24 +47,26 @@ struct FormatCost {
 
 const FormatCost &one_rhs_cost(int prec, int links)
 {
-   static const FormatCost f64 = {{1, 1.05, 0.62, 0.13}, {1, 1.0, 0.90, 0.52}, {3, 1.57, 0.16, 0}};
-   static const FormatCost f32_18 = {{2, 1.02, 0.66, 0.12}, {2, 1.0, 0.51, 0.85}, {4, 1.52, 0.09, 0}};
-   static const FormatCost f32_12 = {{2, 1.13, 0.61, 0.11}, {2, 1.0, 0.97, 0.79}, {4, 1.55, 0.22, 0}};
-   static const FormatCost f16 = {{3, 0.97, 0.50, 0.27}, {2, 1.0, 0.74, 1.15}, {5, 1.10, 0.35, 0}};
+   static const FormatCost f64 = {{1, 1.12, 0.53, 0.54}, {1, 1.0, 0.89, 1.52}, {3, 1.64, 0.07, 0}};
+   static const FormatCost f32_18 = {{2, 0.95, 0.33, 0.19}, {1, 1.0, 0.32, 0.60}, {4, 1.90, 0.52, 0}};
+   static const FormatCost f32_12 = {{2, 1.07, 0.84, 1.12}, {2, 1.0, 0.95, 1.20}, {4, 1.29, 0.39, 0}};
+   static const FormatCost f16 = {{3, 0.83, 0.56, 0.81}, {2, 1.0, 0.78, 1.18}, {5, 1.05, 0.62, 0}};
    return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F16 ? f16 : links == 18 ? f32_18 : f32_12;
 }
 
-const FormatCost &multi_rhs_cost(int prec, int R)  // no tiles
+const FormatCost &multi_rhs_cost(int prec, int links, int R)  // no tiles
 {
    // the t-march (2 and 3 RHS)
-   static const FormatCost f64 = {{1, 1.0, 0.98, 0.74, 32}, {}, {3, 1.35, 0.14, 0}};
-   static const FormatCost f32 = {{2, 1.0, 1.00, 1.44, 32}, {}, {4, 1.35, 0.32, 0}};
-   static const FormatCost f16 = {{3, 1.0, 0.83, 0.45, 12}, {}, {5, 1.30, 0.20, 0}};
+   static const FormatCost f64 = {{1, 1.0, 0.91, 0.43}, {}, {3, 1.58, 0.04, 0}};
+   static const FormatCost f32_18 = {{2, 1.0, 1.00, 0.43}, {}, {4, 1.31, 0.06, 0}};
+   static const FormatCost f32_12 = {{2, 1.0, 1.00, 0.49}, {}, {4, 1.20, 0.09, 0}};
+   static const FormatCost f16 = {{3, 1.0, 1.00, 0.65}, {}, {5, 1.28, 0.53, 0}};
    // the pipelined t-march
    static const FormatCost p64 = {{1, 1.0, 0.99, 0.97, 32}, {}, {3, 1.57, 0.37, 0}};
    static const FormatCost p32 = {{2, 1.0, 0.78, 0.80, 32}, {}, {4, 1.49, 0.39, 0}};
    static const FormatCost p16 = {{3, 1.0, 0.92, 0.20, 12}, {}, {5, 1.40, 0.16, 0}};
-   if (R < kPipeRhs) return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F32 ? f32 : f16;
+   if (R < kPipeRhs)
+      return prec == PLQCD_PREC_F64 ? f64 : prec == PLQCD_PREC_F16 ? f16 : links == 18 ? f32_18 : f32_12;
    return prec == PLQCD_PREC_F64 ? p64 : prec == PLQCD_PREC_F32 ? p32 : p16;
 }
 
@@ -122,16 +125,20 @@ struct Pick {
    const int *L;
    HopTuning best{};
    double cost = 1e300;
-   // `chunk_blocks` blocks per t-chunk, of `lanes` lanes, `per_cu` on a CU
+   // `chunk_blocks` blocks per t-chunk, of `lanes` lanes, `per_cu` on a CU.  Too
+   // few lanes for latency to be hidden at all are left out (10 x 16 x 14 x 54,
+   // F32: 13000 lanes in tiles 45 us, 60000 untiled 15).
    void march(const KernelCost &c, HopTuning t, double chunk_blocks, int lanes, int per_cu)
    {
-      for (int nt = (L[3] + std::min(c.most, L[3]) - 1) / std::min(c.most, L[3]); nt <= L[3];) {
-         const int T = (L[3] + nt - 1) / nt;
+      const bool tile = t.ty > 0;
+      const double fewest = tile ? 16000 : 8000;
+      // the chunk counts that were timed, and one slice per chunk
+      for (int n : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32, 48, 64, L[3]}) {
+         const int nt = std::min(n, L[3]), T = (L[3] + nt - 1) / nt;
+         if (T > c.most || (T > 1 && chunk_blocks * nt * lanes < fewest) || (T == 1 && tile)) continue;
          const double res = double(kCus) * per_cu;
          t.tmarch = T;
-         offer(t, res * lanes * c.k * (T + c.c) * rounds(chunk_blocks * nt, res, c.f));
-         if (T == 1) break;
-         nt = (L[3] + T - 2) / (T - 1);  // the fewest chunks that are shorter
+         offer(t, res * lanes * c.k * (T + c.c) * rounds(chunk_blocks * ((L[3] + T - 1) / T), res, c.f));
       }
    }
    void offer(const HopTuning &t, double v)
@@ -148,19 +155,24 @@ HopTuning pick_shape(const int L[4], int prec, int links, int R, bool solver)
 {
    const int Lxh = L[0] / 2, wave = 64;
    const double S = double(Lxh) * L[1] * L[2], Vh = S * L[3];
-   const FormatCost &fc = R <= 1 ? one_rhs_cost(prec, links) : multi_rhs_cost(prec, R);
+   const FormatCost &fc = R <= 1 ? one_rhs_cost(prec, links) : multi_rhs_cost(prec, links, R);
    Pick p{L};
-   // one RHS: each XCD takes a contiguous eighth; with several an eighth's
-   // slice no longer fits an XCD's L2 and the XCDs sweep the lattice together
-   // (t-march, F64, 12 RHS at 32^3 x 64: 4.2 against 4.5 ms)
+   // Each XCD takes a contiguous eighth; with two or three RHS on large
+   // t-slices the eighth's slices no longer fit an XCD's L2 and the XCDs sweep
+   // the lattice together (F64, mean over the shapes near the best, XCDs
+   // together against eighths: 0.97 at 32^3, 1.01 at 38 x 18 x 26 and 24^3, 1.04
+   // and more below; F32 and F16 alike).
+   const bool together = R > 1 && 2 * S >= 32768;
    for (int block : {64, 128, 256}) {
-      if (R <= 1 ? block != 64 : R < kPipeRhs ? block != 256 : block == 64) continue;
+      if (R <= 1 ? block != 64 : block == 64) continue;
       const int spb = REDUCE_CHUNK * std::max(1, block / (REDUCE_CHUNK * R));
       const int lanes = spb * R, wpb = (lanes + wave - 1) / wave;
-      HopTuning t{R <= 1 ? 1 : 2, R <= 1 ? 1 : 8, block, 0, 1, 0, 0};
+      HopTuning t{together ? 2 : 1, together ? 8 : 1, block, 0, 1, 0, 0};
       const double res = double(kCus) * std::max(1, 4 * fc.gather.waves / wpb);
       const double gb = 2 * std::ceil(Vh / spb);
-      p.offer(t, std::max(gb / res, fc.gather.f) * res * lanes * fc.gather.k);
+      // of equals, gather blocks of 128 lanes (2 RHS at 8^3 x 16: 8.0 against 10.2
+      // us), march blocks of 256
+      p.offer(t, std::max(gb / res, fc.gather.f) * res * lanes * fc.gather.k * (block == 256 ? 1 + 1e-6 : 1));
       int per_cu = 4 * fc.march.waves / wpb;
       if (R >= kPipeRhs) {
          per_cu = std::min<int>(per_cu, 160 * 1024 / pipe_lds(prec, spb));
@@ -169,23 +181,33 @@ HopTuning pick_shape(const int L[4], int prec, int links, int R, bool solver)
       // smaller blocks share each link and halo row among fewer lanes: only
       // where they fit the rounds clearly better
       KernelCost c = fc.march;
-      if (R >= kPipeRhs && block == 128) c.k *= 1.1;
+      if (block == 128) c.k *= R >= kPipeRhs ? 1.1 : 1 + 1e-6;
       p.march(c, t, 2 * std::ceil(S / spb), lanes, std::max(1, per_cu));
    }
    if (R <= 1) {
-      // tiles of 96 lanes or more; of two equally good ones plain H takes the
-      // flatter in y (F64 at 32^3 x 64: 401 us for 32 x 1 x 4, 414 for 32 x 4 x
-      // 1), the solver's epilogues the other (0.0769 against 0.0806 s a solve)
+      // Tiles that fill more than four fifths of 2, 3, 4, 6 or 8 waves (F64 38 x
+      // 18 x 26 x 60, 152 of 192 lanes: 274 us, 228 lanes: 250).  Of equally large ones those longer in y,
+      // within 1 % of the best turn on average (the other way 5 to 7 % above);
+      // except F64 with x rows of 32 sites or more, plain H (401 us for 32 x 1 x 4
+      // at 32^3 x 64, 414 for 32 x 4 x 1; its solver epilogues prefer the long
+      // one too, 0.0769 against 0.0806 s a solve).
+      const bool flat = prec == PLQCD_PREC_F64 && L[0] >= 32 && !solver;
       const int most = prec == PLQCD_PREC_F64 ? 256 : 512;
-      for (int i = 1; i <= L[1] && i * L[0] <= most; i++) {
-         for (int k = 1; k <= L[2] && k * L[0] <= most; k++) {
+      for (int i = 1; i <= 8 && i <= L[1] && i * L[0] <= most; i++) {
+         for (int k = 1; k <= 8 && k <= L[2] && k * L[0] <= most; k++) {
             const int ty = i, tz = k, lanes = L[0] * ty * tz;
-            if (L[1] % ty || L[2] % tz || lanes < 96 || lanes > most) continue;
+            const bool full = (lanes > 102 && lanes <= 128) || (lanes > 153 && lanes <= 192) ||
+                              (lanes > 204 && lanes <= 256) || (lanes > 307 && lanes <= 384) ||
+                              (lanes > 409 && lanes <= 512);
+            if (L[1] % ty || L[2] % tz || !full || lanes > most) continue;
             if (solver && Lxh * ty % REDUCE_CHUNK) continue;  // the norms' chunks
             const int wpb = (lanes + wave - 1) / wave;
             const int per_cu = std::min(4 * fc.tile.waves / wpb, int(160 * 1024 / tile_lds(prec, lanes)));
             KernelCost c = fc.tile;
-            c.k *= 1 + 1e-6 * (solver ? tz : ty);
+            // F64 blocks of up to 128 lanes pass the x links through LDS (32^3 x 64,
+            // 32 x 4 x 1 410 us, 32 x 8 x 1 452)
+            if (prec == PLQCD_PREC_F64 && lanes > 128) c.k *= 1.03;
+            c.k *= 1 + 1e-6 * (flat ? ty : -ty);
             p.march(c, HopTuning{1, 1, 256, 0, 1, ty, tz}, S / (double(Lxh) * ty * tz), lanes, std::max(1, per_cu));
          }
       }

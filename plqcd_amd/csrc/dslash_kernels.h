@@ -1172,6 +1172,162 @@ __global__ __launch_bounds__(BLOCK, pipe_waves<SIO>()) void hop_pipe_kernel(SIO 
    hop_pipe_block<MODE, DAG, EPI, NORM, BLOCK, NIT>(in, out, g, a, logical_block(a), fuse);
 }
 
+// Pipelined t-march for one to three right-hand sides, F64 and F32 18-real:
+// hop_tmarch_kernel's columns, chunks, lanes and order of operations, with
+// every lane's loads (its own links beside the spinors they multiply) issued
+// two neighbours ahead, across the slice boundary too.  With 12-real and F16
+// links the rebuilding and the arithmetic cover more of the latency and the
+// plain t-march holds more waves: it is as fast or up to 6 % faster and stays.
+//   us per H with one RHS, untiled t-march and this: F64 16^3 x 32 30.4 and
+// 26.3, 24^3 x 48 158.7 and 160.5 (its traffic moves at 4.6 TB/s either way);
+// F32 18-real 16^3 x 32 20.9 and 15.8, 20^3 x 40 45.6 and 40.2, 24^3 x 48 87.1
+// and 83.1, 32 x 42 x 24 x 64 241.8 and 227.5.
+template <class SIO, class GIO>
+constexpr bool stream_march()
+{
+   return std::is_same<typename SIO::real, double>::value || (SIO::NC == 6 && std::is_same<GIO, GaugeIO<PLQCD_PREC_F32, 18>>::value);
+}
+template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, class SIO, class GIO, class SO>
+__global__ __launch_bounds__(BLOCK) void hop_stream_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
+{
+   if (NORM && a.halt && *a.halt) return;
+   typedef typename SIO::C C;
+   typedef typename SIO::Sp Sp;
+   typedef typename SIO::Hv Hv;
+   typedef typename GIO::U U;
+   constexpr int SF = DAG ? 1 : -1;
+   constexpr bool compat = MODE == MODE_COMPAT;
+   constexpr int D = 2;  // neighbours in flight
+   const int S = a.S;
+   const int nbS = (S + a.spb - 1) / a.spb;
+   int lb = logical_block(a);
+   const int q = lb & 1;  // parity of the column's first site
+   lb >>= 1;
+   const int sb = lb % nbS;
+   const int chunk = lb / nbS;
+   const int tid = threadIdx.x;
+   const int r = tid % a.R;
+   const int js = tid / a.R;
+   const int rr = rhs_of(a, r);
+   const int c = sb * a.spb + js;
+   const bool valid = c < S;
+   const SIO si = in.at_rhs(rr);
+   const SO so = out.at_rhs(rr);
+   const int t0 = chunk_t0(a, chunk), nts = chunk_t0(a, chunk + 1) - t0;
+   const int Lt = a.L[3];
+   const int cc = valid ? c : 0;
+   const int row = cc / a.Lxh;
+   const int xh = cc - row * a.Lxh;
+   const int y = row % a.L[1];
+   const int z = row / a.L[1];
+   const int odd = (q + y + z + t0) & 1;  // the parity of x, the same at every slice
+   // x neighbours: for odd x, up is xh + 1 and down xh; for even x, up is xh and down xh - 1
+   const int xup = row * a.Lxh + (xh + 1 == a.Lxh ? 0 : xh + 1);
+   const int xdn = row * a.Lxh + (xh == 0 ? a.Lxh - 1 : xh - 1);
+   int cn[6];
+   {
+      cn[0] = odd ? xup : cc;
+      cn[1] = odd ? cc : xdn;
+      const int ryp = (y == a.L[1] - 1) ? row - (a.L[1] - 1) : row + 1;
+      const int rym = (y == 0) ? row + (a.L[1] - 1) : row - 1;
+      const int rzp = (z == a.L[2] - 1) ? row - (a.L[2] - 1) * a.L[1] : row + a.L[1];
+      const int rzm = (z == 0) ? row + (a.L[2] - 1) * a.L[1] : row - a.L[1];
+      cn[2] = ryp * a.Lxh + xh;
+      cn[3] = rym * a.Lxh + xh;
+      cn[4] = rzp * a.Lxh + xh;
+      cn[5] = rzm * a.Lxh + xh;
+   }
+   Sp cen, nxt, ring[D], pre;
+   U lring[D], ut;
+   Hv bt;
+   auto issue = [&](int n, int s) {
+      const int p = q ^ (s & 1), base = (t0 + s) * S;
+      const int col = cn[n];
+      si.load_sps(p ^ 1, col + base, ring[n % D]);
+      if (n & 1) g.template load_raw<false, true>(p ^ 1, n >> 1, col + base, lring[n % D]);
+      else g.template load_raw<false, true>(compat ? 0 : p, n >> 1, cc + base, lring[n % D]);
+   };
+   // prologue as in hop_tmarch_block
+   {
+      const int tm = (t0 == 0 ? Lt : t0) - 1;
+      Sp f;
+      U u;
+      si.load_sps(q ^ 1, cc + tm * S, f);
+      g.template load_raw<false, true>(q ^ 1, 3, cc + tm * S, u);
+      si.load_sps(q, cc + t0 * S, cen);
+#pragma unroll
+      for (int n = 0; n < D; n++) issue(n, 0);
+      GIO::finish(u);
+      term_udag<3, -SF>(f, u, bt);
+   }
+   for (int s = 0; s < nts; s++) {
+      const int t = t0 + s;
+      const int p = q ^ (s & 1);
+      const int base = t * S;
+      const int j = cc + base;
+      const int sn = s + 1 < nts ? s + 1 : s;
+      C acc[12];
+#pragma unroll
+      for (int m = 0; m < 12; m++) acc[m] = C{0, 0};
+      U ub;
+#define PLQCD_PIPE(N, MU)                                                            \
+   {                                                                                 \
+      U u = lring[N % D];                                                            \
+      Hv h;                                                                          \
+      GIO::finish(u);                                                                \
+      if constexpr ((N & 1) == 0) {                                                  \
+         term_u<MU, SF>(ring[N % D], u, h);                                          \
+         accum<MU, SF, !compat>(acc, h);                                             \
+      } else {                                                                       \
+         term_udag<MU, -SF>(ring[N % D], u, h);                                      \
+         accum<MU, -SF, true>(acc, h);                                               \
+      }                                                                              \
+      pin(acc);                                                                      \
+      __builtin_amdgcn_sched_barrier(0);                                             \
+      if (N < 6 - D) issue(N + D, s);                                                \
+      else issue((N + D) % 6, sn);                                                   \
+      __builtin_amdgcn_sched_barrier(0);                                             \
+   }
+      PLQCD_PIPE(0, 0)
+      PLQCD_PIPE(1, 0)
+      PLQCD_PIPE(2, 1)
+      {
+         const int tp = (t + 1 == Lt) ? 0 : t + 1;
+         si.load_sps(p ^ 1, cc + tp * S, nxt);
+         g.template load_raw<true, true>(p, 3, j, ut);  // read by this lane only
+         if constexpr (compat) g.template load_raw<false, true>(0, 3, j, ub);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      PLQCD_PIPE(3, 1)
+   
+      if constexpr (EPI == 3) fuse.p.at_rhs(rr).load_sps(p, j, pre);
+      __builtin_amdgcn_sched_barrier(0);
+      PLQCD_PIPE(4, 2)
+      PLQCD_PIPE(5, 2)
+#undef PLQCD_PIPE
+      {
+         Hv h;
+         GIO::finish(ut);
+         if constexpr (compat) GIO::finish(ub);
+         if constexpr (compat) term_u<3, SF>(nxt, ub, h);
+         else term_u<3, SF>(nxt, ut, h);
+         accum<3, SF, !compat>(acc, h);
+         accum<3, -SF, true>(acc, bt);
+         term_udag<3, -SF>(cen, ut, bt);
+      }
+      double nrm = 0.0;
+      if (valid) {
+         C cv[12];
+         if (EPI >= 1) SIO::to_c(cen, cv);
+         nrm = epilogue<EPI, NORM>(si, so, a, rr, p, j, acc, EPI >= 1 ? cv : (const C *)nullptr, fuse,
+                                   EPI == 3 ? &pre : (const Sp *)nullptr);
+      }
+      cen = nxt;
+      if (NORM) chunk_reduce<BLOCK>(nrm, js, r, a.R, p * a.nchunk + (c + base) / REDUCE_CHUNK, valid,
+                                    a.partial + (size_t)rr * 2 * a.nchunk, s);
+   }
+}
+
 // LDS for the links of a pipelined t-march block (of the CU's 160 KiB)
 constexpr size_t kPipeLds = 144 * 1024;
 // Whether hop_pipe_block runs blocks of `lanes` lanes and spb sites: at most
@@ -1484,8 +1640,12 @@ int launch_one(int variant, dim3 grid, dim3 block, hipStream_t st, S si, SO so, 
          return 0;
       }
    } else if (variant == V_MARCH) {
-      hipLaunchKernelGGL((hop_tmarch_kernel<MODE, DAG, EPI, NORM, BLOCK, S, G, SO>), grid, block, 0, st, si, so, gg, a,
-                         f);
+      if constexpr (stream_march<S, G>())
+         hipLaunchKernelGGL((hop_stream_kernel<MODE, DAG, EPI, NORM, BLOCK, S, G, SO>), grid, block, 0, st, si, so, gg, a,
+                            f);
+      else
+         hipLaunchKernelGGL((hop_tmarch_kernel<MODE, DAG, EPI, NORM, BLOCK, S, G, SO>), grid, block, 0, st, si, so, gg, a,
+                            f);
       return 0;
    } else if (variant == V_TILE) {
       // two LDS buffers of BLOCK spinors, BLOCK half-spinors and (FP64 blocks

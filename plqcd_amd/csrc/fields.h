@@ -41,13 +41,22 @@ __device__ __forceinline__ T ld(const char *ubase, uint32_t off)
 // kernels that load many components at few site offsets in a loop, whose
 // per-lane addresses would otherwise be strength-reduced into two registers
 // for each component and neighbour.  ubase must be wave-uniform.
-template <class T>
+template <class T, bool NT = false>
 __device__ __forceinline__ T ld_s(const char *ubase, uint32_t off)
 {
    typedef const __attribute__((address_space(1))) char *global_ptr;
    global_ptr b = (global_ptr)ubase;
    asm volatile("" : "+s"(b));
-   return *reinterpret_cast<const __attribute__((address_space(1))) T *>(b + off);
+   typedef const __attribute__((address_space(1))) T *global_t;
+   if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<global_t>(b + off));
+   else return *reinterpret_cast<global_t>(b + off);
+}
+// ld or (SB) ld_s
+template <class T, bool NT, bool SB>
+__device__ __forceinline__ T ld_u(const char *ubase, uint32_t off)
+{
+   if constexpr (SB) return ld_s<T, NT>(ubase, off);
+   else return ld<T, NT>(ubase, off);
 }
 template <class T>
 __device__ __forceinline__ void st_nt(char *ubase, uint32_t off, T v)
@@ -375,14 +384,14 @@ struct GaugeIO<PLQCD_PREC_F64, 18> {
    typedef LinkV<C> U;
    const char *base;
    size_t kstride;  // Vh*16: bytes between link components
-   template <bool NT = false>
+   template <bool NT = false, bool SB = false>
    __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
       C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 9 * kstride;
       const uint32_t o = (uint32_t)j * 16;
 #pragma unroll
-      for (int k = 0; k < 9; k++) u[k] = ld<d2, NT>(b + k * kstride, o);
+      for (int k = 0; k < 9; k++) u[k] = ld_u<d2, NT, SB>(b + k * kstride, o);
    }
    static __device__ __forceinline__ void finish(U &) {}
    template <bool NT = false>
@@ -399,14 +408,14 @@ struct GaugeIO<PLQCD_PREC_F64, 12> {
    typedef LinkV<C> U;
    const char *base;
    size_t kstride;
-   template <bool NT = false>
+   template <bool NT = false, bool SB = false>
    __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
       C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 6 * kstride;
       const uint32_t o = (uint32_t)j * 16;
 #pragma unroll
-      for (int k = 0; k < 6; k++) u[k] = ld<d2, NT>(b + k * kstride, o);
+      for (int k = 0; k < 6; k++) u[k] = ld_u<d2, NT, SB>(b + k * kstride, o);
    }
    static __device__ __forceinline__ void finish(U &u) { reconstruct_row2(u.e); }
    template <bool NT = false>
@@ -423,14 +432,14 @@ struct GaugeIO<PLQCD_PREC_F32, 18> {
    typedef LinkV<C> U;
    const char *base;
    size_t kstride;  // Vh*8
-   template <bool NT = false>
+   template <bool NT = false, bool SB = false>
    __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
       C *u = lk.e;
       const char *b = base + (size_t)(parity * 4 + mu) * 9 * kstride;
       const uint32_t o = (uint32_t)j * 8;
 #pragma unroll
-      for (int k = 0; k < 9; k++) u[k] = ld<f2, NT>(b + k * kstride, o);
+      for (int k = 0; k < 9; k++) u[k] = ld_u<f2, NT, SB>(b + k * kstride, o);
    }
    static __device__ __forceinline__ void finish(U &) {}
    template <bool NT = false>
@@ -447,7 +456,7 @@ struct GaugeIO<PLQCD_PREC_F32, 12> {
    typedef LinkV<C> U;
    const char *base;
    size_t kstride;  // Vh*16
-   template <bool NT = false>
+   template <bool NT = false, bool SB = false>
    __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &lk) const
    {
       C *u = lk.e;
@@ -455,7 +464,7 @@ struct GaugeIO<PLQCD_PREC_F32, 12> {
       const uint32_t o = (uint32_t)j * 16;
 #pragma unroll
       for (int k = 0; k < 3; k++) {
-         const f4 v = ld<f4, NT>(b + k * kstride, o);
+         const f4 v = ld_u<f4, NT, SB>(b + k * kstride, o);
          u[2 * k] = f2{v.x, v.y};
          u[2 * k + 1] = f2{v.z, v.w};
       }
@@ -526,12 +535,12 @@ struct GaugeIO<PLQCD_PREC_F16, 12> {
    typedef LinkH U;
    const char *base;  // [parity][mu][Vh] u4 (u00,u01,u02,u10), then [parity][mu][Vh] u2 (u11,u12)
    size_t kstride;    // Vh*16
-   template <bool NT = false>
+   template <bool NT = false, bool SB = false>
    __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &u) const
    {
       const size_t slot = (size_t)(parity * 4 + mu);
-      const u4 a = ld<u4, NT>(base + slot * kstride, (uint32_t)j * 16);
-      const u2 b = ld<u2, NT>(base + 8 * kstride + slot * (kstride / 2), (uint32_t)j * 8);
+      const u4 a = ld_u<u4, NT, SB>(base + slot * kstride, (uint32_t)j * 16);
+      const u2 b = ld_u<u2, NT, SB>(base + 8 * kstride + slot * (kstride / 2), (uint32_t)j * 8);
       u.e[0] = a.x;
       u.e[1] = a.y;
       u.e[2] = a.z;
@@ -554,12 +563,12 @@ struct GaugeIO<PLQCD_PREC_F16, 18> {
    typedef LinkH U;
    const char *base;  // [parity][mu][Vh] u4 (u00..u10), u4 (u11..u21), then [parity][mu][Vh] u32 (u22)
    size_t kstride;    // Vh*16
-   template <bool NT = false>
+   template <bool NT = false, bool SB = false>
    __device__ __forceinline__ void load_raw(int parity, int mu, int j, U &u) const
    {
       const size_t slot = (size_t)(parity * 4 + mu);
-      const u4 a = ld<u4, NT>(base + slot * kstride, (uint32_t)j * 16);
-      const u4 b = ld<u4, NT>(base + (8 + slot) * kstride, (uint32_t)j * 16);
+      const u4 a = ld_u<u4, NT, SB>(base + slot * kstride, (uint32_t)j * 16);
+      const u4 b = ld_u<u4, NT, SB>(base + (8 + slot) * kstride, (uint32_t)j * 16);
       u.e[0] = a.x;
       u.e[1] = a.y;
       u.e[2] = a.z;
@@ -568,7 +577,7 @@ struct GaugeIO<PLQCD_PREC_F16, 18> {
       u.e[5] = b.y;
       u.e[6] = b.z;
       u.e[7] = b.w;
-      u.e[8] = ld<uint32_t, NT>(base + 16 * kstride + slot * (kstride / 4), (uint32_t)j * 4);
+      u.e[8] = ld_u<uint32_t, NT, SB>(base + 16 * kstride + slot * (kstride / 4), (uint32_t)j * 4);
    }
    static __device__ __forceinline__ void finish(U &) {}
    template <bool NT = false>
