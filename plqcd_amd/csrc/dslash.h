@@ -66,17 +66,21 @@ namespace plqcd {
 //                    out = resid_b - (in - kappa H^+ in) for every RHS of the
 //                    launch, stored in out's own precision (any), and its |out|^2
 //                    to partial
+//   kappa_host != null (kappa null): kappa as a host array of the fields' RHS, at
+//                    most kInlineKappa of them, which goes with the launch
 //   halt    != null: (with partial) the launch does nothing when *halt, a device
 //                    flag, is not zero
 //   nr      > 0:     only the right-hand sides r0 .. r0+nr-1 of the fields (kappa,
 //                    alpha and partial stay indexed by the field's RHS)
 //   rlist   != null: only the nr right-hand sides rlist[0 .. nr-1] (a device
 //                    array of distinct RHS of the fields; r0 is not used)
+constexpr int kInlineKappa = 16;
 struct DslashOp {
    int r0 = 0, nr = 0;
    const int *rlist = nullptr;
    int dag = 0;
    const double *kappa = nullptr;
+   const double *kappa_host = nullptr;
    double *partial = nullptr;
    const double *alpha = nullptr;
    const plqcd_hip_field *centre = nullptr;

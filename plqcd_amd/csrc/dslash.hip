@@ -335,9 +335,11 @@ int plqcd::dslash(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip
       return plqcd::set_error(1, "hop: RHS list of %d entries for fields of %d", op.nr, in->nrhs);
    if (!op.rlist && (op.nr < 0 || op.r0 < 0 || (op.nr > 0 && op.r0 + op.nr > in->nrhs)))
       return plqcd::set_error(1, "hop: RHS window %d + %d outside the fields' %d", op.r0, op.nr, in->nrhs);
+   if (op.kappa_host && (op.kappa || in->nrhs > kInlineKappa || op.alpha || op.resid_b || op.partial))
+      return plqcd::set_error(1, "hop: kappa by value is for up to %d right-hand sides of M and M^+", kInlineKappa);
    if (op.centre) {
       const plqcd_hip_field *c = op.centre;
-      if (c->lat != g->lat || c->prec != g->prec || c->nrhs != in->nrhs || c == out || !op.kappa || op.dag ||
+      if (c->lat != g->lat || c->prec != g->prec || c->nrhs != in->nrhs || c == out || !(op.kappa || op.kappa_host) || op.dag ||
           op.alpha || op.partial || op.resid_b)
          return plqcd::set_error(1, "hop: the centre field must be like in, distinct from out, with kappa and no "
                                     "other epilogue");

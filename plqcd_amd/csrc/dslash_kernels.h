@@ -436,6 +436,7 @@ template <class SIO>
 struct CgFuse {
    SIO p;  // EPI 3: b; EPI 4: the centre field
    const double *alpha;
+   double kappa[plqcd::kInlineKappa];  // EPI 1 and 4 without norm: the RHS's kappa where HopArgs::kappa is null
 };
 
 // Epilogue: EPI = 0 stores H in; EPI = 1 stores in(x) - kappa_r * (H in)(x).
@@ -470,7 +471,7 @@ __device__ __forceinline__ double epilogue(const SIO &in, const SO &out, const H
          f.p.at_rhs(r).load(p, j, c0);
       else if (cen == nullptr)
          in.load(p, j, c0);
-      const real kap = (real)a.kappa[r];
+      const real kap = (real)((EPI == 4 || EPI == 1) && !NORM && !a.kappa ? f.kappa[r] : a.kappa[r]);
 #pragma unroll
       for (int m = 0; m < 12; m++) acc[m] = cxmky(cen ? cen[m] : c0[m], kap, acc[m]);
    }
@@ -757,66 +758,19 @@ __device__ __forceinline__ void hop_tmarch_block(const SIO &in, const SO &out, c
       cd[2] = rzm * a.Lxh + xh;
    }
    const int Lt = a.L[3];
-   // The lane's centre spinor and backward t term live across t-slices.  In
-   // the FP64 residual epilogue they stay in LDS (each lane reads only its
-   // own column, so no barrier), which frees 72 registers (226-254 instead of
-   // 256 + 20-38 AGPRs) and lets two blocks share a CU: at 32^3 x 64 with 12
-   // RHS it took 4.1 instead of 5.0 ms.  M (EPI 1) took the same time either
-   // way but, with two blocks per CU sharing the L2, moved 2.77 instead of
-   // 1.81 times its compulsory bytes, and plain H ran 2 % slower, so they and
-   // the other epilogues keep the state in registers, as do FP32 and FP16.
    typedef typename SIO::Sp Sp;
    typedef typename SIO::Hv Hv;
-   constexpr bool CL = std::is_same<typename SIO::real, double>::value && EPI == 3;
-   __shared__ typename Sp::E lcen[CL ? Sp::N : 1][CL ? BLOCK : 1];
-   __shared__ typename Hv::E lbt[CL ? Hv::N : 1][CL ? BLOCK : 1];
-   const int tid = threadIdx.x;
-   Sp cen;
+   Sp cen;  // the lane's centre spinor and backward t term live across t-slices
    Hv b;
-   auto put_cen = [&](const Sp &v) {
-      if constexpr (CL) {
-#pragma unroll
-         for (int m = 0; m < Sp::N; m++) lcen[m][tid] = v.e[m];
-      } else {
-         cen = v;
-      }
-   };
-   auto get_cen = [&](Sp &v) {
-      if constexpr (CL) {
-#pragma unroll
-         for (int m = 0; m < Sp::N; m++) v.e[m] = lcen[m][tid];
-      } else {
-         v = cen;
-      }
-   };
-   auto put_b = [&](const Hv &v) {
-      if constexpr (CL) {
-#pragma unroll
-         for (int m = 0; m < Hv::N; m++) lbt[m][tid] = v.e[m];
-      } else {
-         b = v;
-      }
-   };
-   auto get_b = [&](Hv &v) {
-      if constexpr (CL) {
-#pragma unroll
-         for (int m = 0; m < Hv::N; m++) v.e[m] = lbt[m][tid];
-      } else {
-         v = b;
-      }
-   };
    // prologue: cen = psi(t0); b = U_t(t0-1)^+ (1 -+ g_t) psi(t0-1)
    if (valid) {
-      Sp f, c0;
-      Hv b0;
+      Sp f;
       typename GIO::U u;
-      si.load_sp(q, c + t0 * S, c0);
-      put_cen(c0);
+      si.load_sp(q, c + t0 * S, cen);
       const int tm = (t0 == 0 ? Lt : t0) - 1;
       si.load_sp(q ^ 1, c + tm * S, f);
       g.load_u(q ^ 1, 3, c + tm * S, u);
-      term_udag<3, -SF>(f, u, b0);
-      put_b(b0);
+      term_udag<3, -SF>(f, u, b);
    }
    for (int s = 0; s < nts; s++) {
       const int t = t0 + s;
@@ -834,10 +788,10 @@ __device__ __forceinline__ void hop_tmarch_block(const SIO &in, const SO &out, c
          hop_bwd<1, DAG>(si, g, p, cd[1] + base, acc);
          hop_fwd<2, MODE, DAG>(si, g, p, j, cu[2] + base, acc);
          hop_bwd<2, DAG>(si, g, p, cd[2] + base, acc);
-         Sp f, cs;
+         Sp f;
          {
             typename GIO::U u;
-            Hv rr, bt;
+            Hv rr;
             const int tp = (t + 1 == Lt) ? 0 : t + 1;
             si.load_sp(p ^ 1, c + tp * S, f);
             // U_t(t) serves this slice's forward and the next slice's
@@ -855,20 +809,17 @@ __device__ __forceinline__ void hop_tmarch_block(const SIO &in, const SO &out, c
                term_u<3, SF>(f, u, rr);
             }
             accum<3, SF, MODE != MODE_COMPAT>(acc, rr);
-            get_b(bt);
-            accum<3, -SF, true>(acc, bt);
-            get_cen(cs);
-            term_udag<3, -SF>(cs, u, bt);
-            put_b(bt);
+            accum<3, -SF, true>(acc, b);
+            term_udag<3, -SF>(cen, u, b);
          }
          if (EPI >= 1) {
             C cv[12];
-            SIO::to_c(cs, cv);
+            SIO::to_c(cen, cv);
             nrm = epilogue<EPI, NORM>(si, so, a, rr, p, j, acc, cv, fuse);
          } else {
             nrm = epilogue<EPI, NORM>(si, so, a, rr, p, j, acc, (const C *)nullptr, fuse);
          }
-         put_cen(f);
+         cen = f;
       }
       if (NORM) chunk_reduce<BLOCK>(nrm, js, r, a.R, p * a.nchunk + (sb * a.spb + js + base) / REDUCE_CHUNK, valid,
                                     a.partial + (size_t)rr * 2 * a.nchunk, s);
@@ -1640,7 +1591,7 @@ int launch_one(int variant, dim3 grid, dim3 block, hipStream_t st, S si, SO so, 
          return 0;
       }
    } else if (variant == V_MARCH) {
-      if constexpr (stream_march<S, G>())
+      if constexpr (stream_march<S, G>() && BLOCK <= 256)  // blocks of 512 lanes hold too few registers each
          hipLaunchKernelGGL((hop_stream_kernel<MODE, DAG, EPI, NORM, BLOCK, S, G, SO>), grid, block, 0, st, si, so, gg, a,
                             f);
       else
@@ -1697,7 +1648,7 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
    const int R = op.nr > 0 ? op.nr : in->nrhs;
    a.r0 = op.nr > 0 && !op.rlist ? op.r0 : 0;
    a.rlist = op.rlist;
-   const bool solver = op.kappa != nullptr;
+   const bool solver = op.kappa || op.kappa_host;  // M or M^+
    HopTuning tu = plqcd::default_tuning(lat->L, PREC, LINKS, R, solver);
    plqcd::lookup_tuning(plqcd::TuneKey{{lat->L[0], lat->L[1], lat->L[2], lat->L[3]}, PREC, LINKS, R,
                                        solver ? plqcd::kTuneOpSolver : plqcd::kTuneOpHop},
@@ -1723,17 +1674,19 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
    a.halt = op.halt;
    a.nchunk = plqcd::reduce_chunks(lat->Vh);
    const bool dag = op.dag != 0;
-   const int epi = resid ? 3 : op.alpha ? 2 : op.centre ? 4 : op.kappa ? 1 : 0;
+   const int epi = resid ? 3 : op.alpha ? 2 : op.centre ? 4 : solver ? 1 : 0;
    const bool norm = op.partial != nullptr;
    if ((dag || epi || norm) && mode != PLQCD_HOP_WILSON)
       return plqcd::set_error(2, "hop: M, M^+ and norms need the wilson mode");
    if (epi == 2 && (!dag || !norm || !op.kappa))
       return plqcd::set_error(2, "hop: the CG-update epilogue needs M^+, a norm and kappa");
-   if (epi == 4 && (dag || norm || !op.kappa))
+   if (epi == 4 && (dag || norm || !solver))
       return plqcd::set_error(2, "hop: the external-centre epilogue needs kappa, and no M^+ or norm");
    if (epi == 3 && (PREC != PLQCD_PREC_F64 || !dag || !norm || !op.kappa))
       return plqcd::set_error(2, "hop: the residual epilogue needs F64 storage, M^+, a norm and kappa");
    CgFuse<S> fu{};
+   if (op.kappa_host)
+      for (int r = 0; r < in->nrhs; r++) fu.kappa[r] = op.kappa_host[r];
    if (epi == 2) {
       fu.alpha = op.alpha;
    } else if (epi == 4) {
@@ -1823,13 +1776,13 @@ int launch_t(const plqcd_hip_gauge *g, const plqcd_hip_field *in, plqcd_hip_fiel
       if (epi == 0) lrc = launch_block<PLQCD_HOP_WILSON, false, 0, false>(mblock, variant, grid, block, st, si, so, gg, a);
       else if (epi == 4)
          lrc = launch_block<PLQCD_HOP_WILSON, false, 4, false>(mblock, variant, grid, block, st, si, so, gg, a, fu);
-      else if (!norm) lrc = launch_block<PLQCD_HOP_WILSON, false, 1, false>(mblock, variant, grid, block, st, si, so, gg, a);
+      else if (!norm) lrc = launch_block<PLQCD_HOP_WILSON, false, 1, false>(mblock, variant, grid, block, st, si, so, gg, a, fu);
       else lrc = launch_block<PLQCD_HOP_WILSON, false, 1, true>(mblock, variant, grid, block, st, si, so, gg, a);
    } else {
       if (epi == 0) lrc = launch_block<PLQCD_HOP_WILSON, true, 0, false>(mblock, variant, grid, block, st, si, so, gg, a);
       else if (epi == 2)
          lrc = launch_block<PLQCD_HOP_WILSON, true, 2, true>(mblock, variant, grid, block, st, si, so, gg, a, fu);
-      else if (!norm) lrc = launch_block<PLQCD_HOP_WILSON, true, 1, false>(mblock, variant, grid, block, st, si, so, gg, a);
+      else if (!norm) lrc = launch_block<PLQCD_HOP_WILSON, true, 1, false>(mblock, variant, grid, block, st, si, so, gg, a, fu);
       else lrc = launch_block<PLQCD_HOP_WILSON, true, 1, true>(mblock, variant, grid, block, st, si, so, gg, a);
    }
    if (lrc) return lrc;

@@ -160,3 +160,25 @@ def test_iterations_enqueued_ahead(hp, prec, links):
             s1 = solver.cg_solve(g, b1, x1, 0.12, tol[r], max_iter=most, sloppy=gs)[0]
             assert s1["iterations"] == st[r]["iterations"]
             assert np.array_equal(x1.download(), x.download(r))
+
+
+@pytest.mark.parametrize("R", [1, 16, 17, 40])
+def test_kappa_with_the_launch_and_from_memory(hp, R):
+    """M, M^+ and the Schur operator with as many kappas as travel with a launch
+    and one more: every RHS is bitwise its own one-RHS call."""
+    from plqcd_amd import solver
+    L = (4, 6, 4, 6)
+    lat, g, fi, fo, qs, u = fields(hp, L, hp.PREC_F64, 18, R)
+    ft = hp.Field(lat, hp.PREC_F64, R)
+    f1, o1, t1 = hp.Field(lat), hp.Field(lat), hp.Field(lat)
+    kap = [0.1 + 0.001 * r for r in range(R)]
+    half = len(qs[0]) // 2
+    for dagger in (False, True):
+        solver.apply_m(g, fi, fo, kap, dagger)
+        for r in (0, R // 2, R - 1):
+            solver.apply_m(g, f1.upload(qs[r]), o1, kap[r], dagger)
+            assert np.array_equal(fo.download(r), o1.download()), (dagger, r)
+    solver.apply_schur(g, fi, ft, fo, kap, 1)
+    for r in (0, R // 2, R - 1):
+        solver.apply_schur(g, f1.upload(qs[r]), t1, o1, kap[r], 1)
+        assert np.array_equal(fo.download(r)[half:], o1.download()[half:]), r
