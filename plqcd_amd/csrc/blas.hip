@@ -189,8 +189,7 @@ __global__ __launch_bounds__(256) void k_reduce_fin(const double *partial, size_
 // block of RHS r that finishes its segment last (count[r] says which), then
 //   OP 0:  pap = sum, alpha = rr / pap
 //   OP 1:  rr_new = sum, beta = rr_new / rr, rr_prev = rr, rr = rr_new
-// as k_alpha and k_beta in solver.hip compute them.  The segment sums cross
-// XCDs inside the launch: device-scope atomics.  An iteration takes 5 launches
+// The segment sums cross XCDs inside the launch: device-scope atomics.  An iteration takes 5 launches
 // instead of 9, each of which costs 2 to 6 us however little it does (FP64 one
 // RHS 16^3 x 32: 8 us less an iteration of 150; 8^3 x 16: 3.5 less of 58).
 template <int OP>

@@ -1555,11 +1555,11 @@ __global__ __launch_bounds__(BLOCK) void hop_tile_kernel(SIO in, SIO out, GIO g,
    }
 }
 
-// kernel variants: gather (1 RHS per lane), t-march, RHS-blocked gather, LDS tile, pipelined t-march
+// kernel variants: gather (1 RHS per lane), t-march, RHS-blocked gather, LDS tile, pipelined t-march, half lattice
 enum Variant { V_GATHER = 0, V_MARCH = 1, V_RB2 = 2, V_RB4 = 4, V_TILE = 8, V_PIPE = 16, V_HALF = 32 };
 
 // S: the input field's accessor; SO: the output's (differs only with EPI 3,
-// which runs the gather kernel).  Returns 0 when the kernel was enqueued, and
+// which the tile and RHS-blocked kernels don't have).  Returns 0 when the kernel was enqueued, and
 // an error when the variant does not exist for these template arguments (the
 // host-side checks of launch_t keep such launches out; this keeps a future
 // change from silently launching nothing).
