@@ -57,10 +57,10 @@ const FormatCost &one_rhs_cost(int prec, int links)
 const FormatCost &multi_rhs_cost(int prec, int links, int R)  // no tiles
 {
    // the t-march (2 and 3 RHS)
-   static const FormatCost f64 = {{1, 1.0, 0.91, 0.43}, {}, {3, 1.58, 0.04, 0}};
+   static const FormatCost f64 = {{1, 1.0, 0.91, 0.43, 32}, {}, {3, 1.58, 0.04, 0}};
    static const FormatCost f32_18 = {{2, 1.0, 1.00, 0.43}, {}, {4, 1.31, 0.06, 0}};
    static const FormatCost f32_12 = {{2, 1.0, 1.00, 0.49}, {}, {4, 1.20, 0.09, 0}};
-   static const FormatCost f16 = {{3, 1.0, 1.00, 0.65}, {}, {5, 1.28, 0.53, 0}};
+   static const FormatCost f16 = {{3, 1.0, 1.00, 0.65, 8}, {}, {5, 1.28, 0.53, 0}};
    // the pipelined t-march
    static const FormatCost p64 = {{1, 1.0, 0.99, 0.97, 32}, {}, {3, 1.57, 0.37, 0}};
    static const FormatCost p32 = {{2, 1.0, 0.78, 0.80, 32}, {}, {4, 1.49, 0.39, 0}};
@@ -159,10 +159,14 @@ HopTuning pick_shape(const int L[4], int prec, int links, int R, bool solver)
    Pick p{L};
    // Each XCD takes a contiguous eighth; with two or three RHS on large
    // t-slices the eighth's slices no longer fit an XCD's L2 and the XCDs sweep
-   // the lattice together (F64, mean over the shapes near the best, XCDs
-   // together against eighths: 0.97 at 32^3, 1.01 at 38 x 18 x 26 and 24^3, 1.04
-   // and more below; F32 and F16 alike).
-   const bool together = R > 1 && 2 * S >= 32768;
+   // the lattice together (mean over the shapes near the best, XCDs together
+   // against eighths: 0.97 at 32^3, 1.01 at 38 x 18 x 26 and 24^3, 1.04 and more
+   // below).  F64 with two RHS from somewhat larger ones on (us, 32^3 x 64 785
+   // and 771, 40^3 x 80 1951 and 1987; three RHS at 32^3 x 64 1129 and 1159); F16,
+   // a quarter of the bytes, never (two RHS 190 and 184, at 40^3 x 80 450 and 444;
+   // three 279 and 273).
+   const bool together = R > 1 && prec != PLQCD_PREC_F16 &&
+                         2 * S * (prec == PLQCD_PREC_F64 ? R : 3) >= 3 * 32768;
    for (int block : {64, 128, 256}) {
       if (R <= 1 ? block != 64 : block == 64) continue;
       const int spb = REDUCE_CHUNK * std::max(1, block / (REDUCE_CHUNK * R));
@@ -175,12 +179,26 @@ HopTuning pick_shape(const int L[4], int prec, int links, int R, bool solver)
       p.offer(t, std::max(gb / res, fc.gather.f) * res * lanes * fc.gather.k * (block == 256 ? 1 + 1e-6 : 1));
       int per_cu = 4 * fc.march.waves / wpb;
       if (R >= kPipeRhs) {
+         // F16 with the solver's epilogues and two links per lane: two waves (pipe_waves)
+         if (solver && prec == PLQCD_PREC_F16 && 7 * spb > lanes) per_cu = 4 * 2 / wpb;
          per_cu = std::min<int>(per_cu, 160 * 1024 / pipe_lds(prec, spb));
          pick_patch(L, prec, spb, &t);
       }
       // smaller blocks share each link and halo row among fewer lanes: only
       // where they fit the rounds clearly better
       KernelCost c = fc.march;
+      // one RHS in F16: long marches drift apart, the solver's epilogues sooner (us
+      // per H with 12, 16, 24 and 96 slices, 48^3 x 96: 529, 538, 544, 566; ms per
+      // CG solve with 8, 12, 16 and 32: 26.9, 27.4, 29.4, 35.7 at 32^3 x 64).  Those
+      // epilogues also hold fewer waves (6 slices, which would fill three waves
+      // best: 28.5) and fill a round sooner (24^3 x 48, 6 and 8 slices: 11.9, 12.7)
+      if (R <= 1 && prec == PLQCD_PREC_F16) {
+         c.most = solver ? 8 : 16;
+         if (solver) {
+            per_cu = 4 * 2 / wpb;
+            c.f = 0.8;
+         }
+      }
       if (block == 128) c.k *= R >= kPipeRhs ? 1.1 : 1 + 1e-6;
       p.march(c, t, 2 * std::ceil(S / spb), lanes, std::max(1, per_cu));
    }

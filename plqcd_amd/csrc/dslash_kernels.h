@@ -1110,14 +1110,17 @@ __device__ __forceinline__ void hop_pipe_block(const SIO &in, const SO &out, con
 
 // Waves a SIMD is to hold.  F16 with the solver's epilogues takes 174 to 192
 // registers by itself, two waves; held to three it spills 6 to 25 (12 RHS at
-// 24^3 x 48: M 375 -> 360 us, M^+ with the update 410 -> 394).
-template <class SIO>
+// 24^3 x 48: M 375 -> 360 us, M^+ with the update 410 -> 394).  With two links
+// per lane and slice (four to six RHS) it would spill 30 to 34, and two waves
+// are the faster: a 4-RHS CG 97.3 -> 84.0 ms at 32^3 x 64, 243.9 -> 212.2 at
+// 40^3 x 80 (the plain t-march 86.2 and 213.3).
+template <class SIO, int EPI, int NIT>
 constexpr int pipe_waves()
 {
-   return std::is_same<typename SIO::real, double>::value ? 1 : SIO::NC == 6 ? 2 : 3;
+   return std::is_same<typename SIO::real, double>::value ? 1 : SIO::NC == 6 ? 2 : EPI >= 1 && NIT > 1 ? 2 : 3;
 }
 template <int MODE, bool DAG, int EPI, bool NORM, int BLOCK, int NIT, class SIO, class GIO, class SO>
-__global__ __launch_bounds__(BLOCK, pipe_waves<SIO>()) void hop_pipe_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
+__global__ __launch_bounds__(BLOCK, (pipe_waves<SIO, EPI, NIT>())) void hop_pipe_kernel(SIO in, SO out, GIO g, HopArgs a, CgFuse<SIO> fuse)
 {
    if (NORM && a.halt && *a.halt) return;
    hop_pipe_block<MODE, DAG, EPI, NORM, BLOCK, NIT>(in, out, g, a, logical_block(a), fuse);
